@@ -19,13 +19,9 @@
 // Results equal the real-transform derivatives to rounding.
 //
 // When an axis length factors into 2, 3, 5, 7, 11 and 13, its derivatives
-// skip hipFFT: one pstd_dfft launch takes every derivative of a stage along
-// that axis.  A workgroup loads a tile of row pairs (z) or column pairs (x)
-// into LDS as complex numbers, runs a mixed-radix Stockham FFT in LDS,
-// multiplies by the whole-spectrum multiplier, runs the inverse as the
-// conjugate of the forward transform of the conjugate, and writes the two
-// derivatives: one HBM read and one write per value instead of six
-// (forward transform, multiplier pass, inverse transform).
+// skip hipFFT: one pstd_dfft launch (pstd_fft.hpp) takes every derivative of
+// a stage along both axes, with one read and one write per value instead of
+// six (forward transform, multiplier pass, inverse transform).
 //
 // CPML (pml.c:1959-2106): per stage (fp1, fp23, fp4) and axis the rows b,
 // c at nodes, bh, ch at inner half nodes, bH, cH at outer half nodes; the
@@ -51,15 +47,11 @@
 #include <cmath>
 #include <vector>
 
+#include "pstd_fft.hpp"
 #include "sm_internal.hpp"
 
 namespace sm {
 namespace pstd {
-
-template <typename T>
-struct Cx {
-    T re, im;
-};
 
 // CPML table rows per stage and axis, then shared k rows per axis
 enum { T_B, T_C, T_BH, T_CH, T_BHE, T_CHE, T_NST };
@@ -81,13 +73,11 @@ struct Grid {
     sm_dbuf tabs;                   // per stage 2 x T_NST rows, then 2 x K_NK rows (np + 1 each)
     size_t kx_n = 0;                // entries per x multiplier row (nx2 paired, nxh otherwise)
     hipfftHandle px_f = 0, px_i = 0, pz_f = 0, pz_i = 0;
-    // hand-written transforms per axis (0 x, 1 z): radices packed 4 bits a
-    // pass (index into FFT_RADICES), pairs per workgroup, twiddles
-    // e^{-2 pi i k/n} and whole-spectrum multipliers (fwd then bwd)
+    // hand-written transforms per axis (0 x, 1 z): plan, twiddles and
+    // whole-spectrum multipliers (fwd then bwd)
     bool own[2] = {false, false};
-    int nr[2] = {0, 0};
-    uint64_t rcode[2] = {0, 0};
-    int P[2] = {1, 1};
+    FftPlan fft[2];
+    int cus = 256;                  // compute units of the device
     sm_dbuf tw[2], fmul[2];
 };
 
@@ -200,323 +190,6 @@ int deriv(Grid &g, const T *f, int axis, bool fwd, T *out)
     return SM_OK;
 }
 
-// ------------------------------------------------------------------
-// hand-written FFT derivatives
-// ------------------------------------------------------------------
-constexpr int FFT_MAXPASS = 12;
-constexpr int FFT_RADICES[9] = {2, 3, 4, 5, 7, 8, 11, 13, 16};
-
-// radices of n, largest powers of two first; false if n has another factor
-inline bool fft_factor(int n, int &nr, uint64_t &code)
-{
-    nr = 0;
-    code = 0;
-    int m = n;
-    auto push = [&](int r) {
-        int q = 0;
-        while (FFT_RADICES[q] != r) ++q;
-        code |= (uint64_t)q << (4 * nr);
-        ++nr;
-    };
-    // odd radices first: the first Stockham pass writes with a stride of R
-    // elements, which for a power of two puts a wave's lanes on a few LDS
-    // banks; later passes write runs of Ns consecutive elements
-    int two = 0;
-    while (m % 2 == 0) { m /= 2; ++two; }
-    for (int r : {13, 11, 7, 5, 3})
-        while (m % r == 0) {
-            if (nr >= FFT_MAXPASS) return false;
-            push(r);
-            m /= r;
-        }
-    if (two % 4 == 3) push(8);
-    else if (two % 4 == 2) push(4);
-    else if (two % 4 == 1) push(2);
-    for (int q = 0; q < two / 4; ++q) {
-        if (nr >= FFT_MAXPASS) return false;
-        push(16);
-    }
-    return m == 1 && n >= 2 && nr > 0 && nr <= FFT_MAXPASS;
-}
-
-// a b + c with one rounding
-__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double mad(double a, double b, double c) { return __builtin_fma(a, b, c); }
-
-template <typename T>
-__device__ __forceinline__ Cx<T> cmul(Cx<T> a, Cx<T> b)
-{
-    // fused multiply-adds: one rounding less per product (the transforms
-    // are held to a tolerance, not to the reference's FFTW bits)
-    return {mad(a.re, b.re, -(a.im * b.im)), mad(a.re, b.im, a.im * b.re)};
-}
-template <typename T>
-__device__ __forceinline__ Cx<T> cadd(Cx<T> a, Cx<T> b) { return {a.re + b.re, a.im + b.im}; }
-template <typename T>
-__device__ __forceinline__ Cx<T> csub(Cx<T> a, Cx<T> b) { return {a.re - b.re, a.im - b.im}; }
-// -i a
-template <typename T>
-__device__ __forceinline__ Cx<T> cmi(Cx<T> a) { return {a.im, -a.re}; }
-
-// forward DFT of v[0..R) in place, w = e^{-2 pi i / R} = r[rs] (r holds
-// the roots of unity of the pass's radix; rs > 1 inside a larger radix)
-template <typename T, int R>
-__device__ __forceinline__ void dft(Cx<T> *v, const Cx<T> *r, int rs)
-{
-    if constexpr (R == 2) {
-        const Cx<T> a = v[0], b = v[1];
-        v[0] = cadd(a, b); v[1] = csub(a, b);
-    } else if constexpr (R == 4) {
-        const Cx<T> a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]), a2 = cadd(v[1], v[3]), a3 = csub(v[1], v[3]);
-        v[0] = cadd(a0, a2); v[2] = csub(a0, a2);
-        v[1] = cadd(a1, cmi(a3)); v[3] = csub(a1, cmi(a3));
-    } else if constexpr (R == 8 || R == 16) {
-        // two half-length DFTs of the even and odd samples, combined with
-        // w^k (from the table)
-        constexpr int H = R / 2;
-        Cx<T> e[H], o[H];
-#pragma unroll
-        for (int t = 0; t < H; ++t) { e[t] = v[2 * t]; o[t] = v[2 * t + 1]; }
-        dft<T, H>(e, r, 2 * rs);
-        dft<T, H>(o, r, 2 * rs);
-#pragma unroll
-        for (int k = 0; k < H; ++k) {
-            const Cx<T> wo = k == 0 ? o[k] : cmul(o[k], r[k * rs]);
-            v[k] = cadd(e[k], wo);
-            v[k + H] = csub(e[k], wo);
-        }
-    } else {
-        // odd R: pair t with R - t; X_s = A_s - i B_s, X_{R-s} = A_s + i B_s
-        // with A_s = v0 + sum (v_t + v_{R-t}) cos, B_s = sum (v_t - v_{R-t}) sin
-        constexpr int H = (R - 1) / 2;
-        Cx<T> sp[H], sm[H];
-        Cx<T> x0 = v[0];
-#pragma unroll
-        for (int t = 1; t <= H; ++t) {
-            sp[t - 1] = cadd(v[t], v[R - t]);
-            sm[t - 1] = csub(v[t], v[R - t]);
-            x0 = cadd(x0, sp[t - 1]);
-        }
-        Cx<T> out[R];
-        out[0] = x0;
-#pragma unroll
-        for (int s = 1; s <= H; ++s) {
-            Cx<T> A = v[0], B = {T(0), T(0)};
-#pragma unroll
-            for (int t = 1; t <= H; ++t) {
-                const Cx<T> w = r[((s * t) % R) * rs];   // (cos, -sin)
-                A.re = mad(sp[t - 1].re, w.re, A.re); A.im = mad(sp[t - 1].im, w.re, A.im);
-                B.re = mad(-sm[t - 1].re, w.im, B.re); B.im = mad(-sm[t - 1].im, w.im, B.im);
-            }
-            out[s] = {A.re + B.im, A.im - B.re};
-            out[R - s] = {A.re - B.im, A.im + B.re};
-        }
-#pragma unroll
-        for (int t = 0; t < R; ++t) v[t] = out[t];
-    }
-}
-
-// where a pass reads and writes: the LDS buffers (transform p at p ls), or,
-// for the first forward and the last inverse pass, the field f and the
-// derivative out in global memory (pair p: rows or columns r0, r0 + 1 with
-// r0 = r0base + 2p, a missing partner read as 0 and not written); with mul,
-// the pass writes conj(mul[k] v) (the multiplier between the transforms)
-template <typename T>
-struct PassIO {
-    const Cx<T> *src;
-    Cx<T> *dst;
-    const T *f;
-    T *out;
-    const Cx<T> *mul;
-    int ls, r0base, lim, nz2;
-    bool in_g, out_g;
-};
-
-template <typename T, int AX>
-__device__ __forceinline__ Cx<T> gload(const PassIO<T> io, int p, int k)
-{
-    const int r0 = io.r0base + 2 * p;
-    T re = T(0), im = T(0);
-    if (AX == 1) {
-        if (r0 < io.lim) re = io.f[(size_t)r0 * io.nz2 + k];
-        if (r0 + 1 < io.lim) im = io.f[(size_t)(r0 + 1) * io.nz2 + k];
-    } else {
-        if (r0 < io.lim) re = io.f[(size_t)k * io.nz2 + r0];
-        if (r0 + 1 < io.lim) im = io.f[(size_t)k * io.nz2 + r0 + 1];
-    }
-    return {re, im};
-}
-
-template <typename T, int AX>
-__device__ __forceinline__ void gstore(const PassIO<T> io, int p, int k, Cx<T> y)
-{
-    const int r0 = io.r0base + 2 * p;
-    if (AX == 1) {
-        if (r0 < io.lim) io.out[(size_t)r0 * io.nz2 + k] = y.re;
-        if (r0 + 1 < io.lim) io.out[(size_t)(r0 + 1) * io.nz2 + k] = -y.im;
-    } else {
-        if (r0 < io.lim) io.out[(size_t)k * io.nz2 + r0] = y.re;
-        if (r0 + 1 < io.lim) io.out[(size_t)k * io.nz2 + r0 + 1] = -y.im;
-    }
-}
-
-// one Stockham pass of radix R over P transforms of length n; Ns = product
-// of the earlier radices; twp[(t - 1) Ns + k] = e^{-2 pi i k t / (Ns R)}
-// (consecutive k on consecutive LDS banks), roots the R-th roots of unity.
-// Passes that touch global memory along x take the pairs fastest (2P
-// adjacent values of a row per lane group).
-template <typename T, int R, int AX>
-__device__ __forceinline__ void fft_pass(const PassIO<T> io, int n, int P, int Ns, const Cx<T> *twp,
-                                         const Cx<T> *roots)
-{
-    const int nb = n / R, ls = io.ls;
-    const bool pf = AX == 0 && (io.in_g || io.out_g);
-    for (int l = threadIdx.x; l < nb * P; l += blockDim.x) {
-        int p, j;
-        if (pf) { j = l / P; p = l - j * P; }
-        else { p = l / nb; j = l - p * nb; }
-        const int k = j % Ns;
-        Cx<T> v[R];
-        if (io.in_g) {
-#pragma unroll
-            for (int t = 0; t < R; ++t) v[t] = gload<T, AX>(io, p, j + t * nb);
-        } else {
-            const Cx<T> *s = io.src + p * ls;
-#pragma unroll
-            for (int t = 0; t < R; ++t) v[t] = s[j + t * nb];
-        }
-        if (k) {
-#pragma unroll
-            for (int t = 1; t < R; ++t) v[t] = cmul(v[t], twp[(t - 1) * Ns + k]);
-        }
-        dft<T, R>(v, roots, 1);
-        const int base = (j - k) * R + k;
-        if (io.mul) {
-#pragma unroll
-            for (int t = 0; t < R; ++t) {
-                const Cx<T> z = cmul(v[t], io.mul[base + t * Ns]);
-                v[t] = {z.re, -z.im};
-            }
-        }
-        if (io.out_g) {
-#pragma unroll
-            for (int t = 0; t < R; ++t) gstore<T, AX>(io, p, base + t * Ns, v[t]);
-        } else {
-            Cx<T> *d = io.dst + p * ls;
-#pragma unroll
-            for (int t = 0; t < R; ++t) d[base + t * Ns] = v[t];
-        }
-    }
-}
-
-// a forward FFT of P transforms: from global memory (in_g) or LDS buffer a
-// (scratch b), into LDS (returned, after a barrier) or global memory
-// (out_g), the last pass applying mul if given.  Inlined: an out-of-line
-// call would keep a stack frame in scratch memory.
-template <typename T, int AX>
-__device__ __forceinline__ Cx<T> *fft_run(PassIO<T> io, Cx<T> *a, Cx<T> *b, int n, int P, int nr, uint64_t code,
-                                          const Cx<T> *tw, bool in_g, bool out_g, const Cx<T> *mul)
-{
-    int Ns = 1;
-    for (int q = 0; q < nr; ++q) {
-        const int ri = (int)((code >> (4 * q)) & 15);
-        const int R = FFT_RADICES[ri];
-        const Cx<T> *roots = tw + (R - 1) * Ns;
-        io.src = a;
-        io.dst = b;
-        io.in_g = in_g && q == 0;
-        io.out_g = out_g && q == nr - 1;
-        io.mul = q == nr - 1 ? mul : nullptr;
-        switch (ri) {
-        case 0: fft_pass<T, 2, AX>(io, n, P, Ns, tw, roots); break;
-        case 1: fft_pass<T, 3, AX>(io, n, P, Ns, tw, roots); break;
-        case 2: fft_pass<T, 4, AX>(io, n, P, Ns, tw, roots); break;
-        case 3: fft_pass<T, 5, AX>(io, n, P, Ns, tw, roots); break;
-        case 4: fft_pass<T, 7, AX>(io, n, P, Ns, tw, roots); break;
-        case 5: fft_pass<T, 8, AX>(io, n, P, Ns, tw, roots); break;
-        case 6: fft_pass<T, 11, AX>(io, n, P, Ns, tw, roots); break;
-        case 7: fft_pass<T, 13, AX>(io, n, P, Ns, tw, roots); break;
-        default: fft_pass<T, 16, AX>(io, n, P, Ns, tw, roots); break;
-        }
-        tw = roots + R;   // the next pass's table
-        Ns *= R;
-        if (!io.out_g) __syncthreads();
-        Cx<T> *t = a; a = b; b = t;
-    }
-    return a;
-}
-
-// up to 8 derivatives of one stage along one axis: job j differentiates
-// field ((fields >> 4j) & 15) of x into d + ((slots >> 4j) & 15) N, with
-// the forward multiplier if bit j of fwd is set
-template <typename T>
-struct DfftArgs {
-    const T *x;
-    T *d;
-    unsigned N;
-    uint32_t fields, slots, fwd;
-    int njobs;
-    const Cx<T> *tw, *mul_f, *mul_b;
-    int n, nr, tsz;
-    uint64_t code;
-    int nx2, nz2;
-    int P, ntiles, nblocks;
-};
-
-extern __shared__ __align__(16) unsigned char pstd_lds[];
-
-// AX 1: z (unit stride), row pairs (r, r + 1); AX 0: x (stride nz2),
-// column pairs (c, c + 1); a missing partner reads as 0 and is not written.
-// b: the workgroup's tile of this axis's jobs
-template <typename T, int AX>
-__device__ __forceinline__ void dfft_body(const DfftArgs<T> &a, int b)
-{
-    const int jb = b / a.ntiles, tile = b - jb * a.ntiles;
-    const T *f = a.x + (size_t)((a.fields >> (4 * jb)) & 15) * a.N;
-    T *out = a.d + (size_t)((a.slots >> (4 * jb)) & 15) * a.N;
-    const Cx<T> *mul = ((a.fwd >> jb) & 1) ? a.mul_f : a.mul_b;
-    const int n = a.n, P = a.P, ls = n + 1;
-    // LDS: two buffers of P transforms (stride n + 1), then the per-pass
-    // twiddles and roots
-    Cx<T> *A = (Cx<T> *)pstd_lds, *B = A + P * ls, *tw = B + P * ls;
-    for (int l = threadIdx.x; l < a.tsz; l += blockDim.x) tw[l] = a.tw[l];
-    __syncthreads();
-    PassIO<T> io;
-    io.f = f; io.out = out; io.ls = ls; io.r0base = 2 * tile * P;
-    io.lim = AX == 1 ? a.nx2 : a.nz2; io.nz2 = a.nz2;
-    // Z = DFT(f) from global memory, written as conj(M Z); y = IDFT(M Z) =
-    // conj(DFT(conj(M Z))) into global memory (one call site: inlined once)
-    Cx<T> *c = A;
-    for (int rep = 0; rep < 2; ++rep)
-        c = fft_run<T, AX>(io, c, c == A ? B : A, n, P, a.nr, a.code, tw, rep == 0, rep == 1,
-                           rep == 0 ? mul : nullptr);
-}
-
-// workgroups of one XCD take consecutive tiles (adjacent columns share
-// cache lines)
-__device__ __forceinline__ int xcd_tile(int nblocks)
-{
-    const int per = (nblocks + 7) / 8;
-    return (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-}
-
-template <typename T, int AX>
-__global__ __launch_bounds__(512) void pstd_dfft(const DfftArgs<T> a)
-{
-    const int b = xcd_tile(a.nblocks);
-    if (b < a.nblocks) dfft_body<T, AX>(a, b);
-}
-
-// the derivatives of a stage along x (ax) and z (az) in one grid: the x
-// tiles first, then the z tiles
-template <typename T>
-__global__ __launch_bounds__(512) void pstd_dfft_xz(const DfftArgs<T> ax, const DfftArgs<T> az)
-{
-    const int b = xcd_tile(ax.nblocks + az.nblocks);
-    if (b < ax.nblocks) dfft_body<T, 0>(ax, b);
-    else if (b < ax.nblocks + az.nblocks) dfft_body<T, 1>(az, b - ax.nblocks);
-}
-
 // sources the stage kernels inject themselves, after the update of their
 // cell (at most SRC_FUSED: more go through the solver's separate
 // one-thread source kernel): cell[s] of source s; type, cell, offset and
@@ -538,37 +211,53 @@ struct DJob {
     bool fwd;
 };
 
-// complex entries of the per-pass tables: (R - 1) Ns twiddles and R roots
-inline int tw_count(int nr, uint64_t code)
+// pairs per thread (V) and groups of V pairs per workgroup (P) of a launch of
+// nx derivatives along x and nz along z
+struct FftShape {
+    int V, P;
+};
+inline FftShape fft_shape(const Grid &g, size_t elt, int nx, int nz)
 {
-    int c = 0, Ns = 1;
-    for (int q = 0; q < nr; ++q) {
-        const int R = FFT_RADICES[(code >> (4 * q)) & 15];
-        c += (R - 1) * Ns + R;
-        Ns *= R;
+    const int count[2] = {nx, nz}, lines[2] = {g.nz2, g.nx2};
+    auto blocks = [&](int V, int P) {
+        int b = 0;
+        for (int ax = 0; ax < 2; ++ax) b += count[ax] * ((lines[ax] + 2 * V * P - 1) / (2 * V * P));
+        return b;
+    };
+    auto fits = [&](int V, int P) {
+        for (int ax = 0; ax < 2; ++ax)
+            if (count[ax] && (fft_lds(g.fft[ax], V, P, elt) > 81920 || fft_threads(g.fft[ax], P) > FFT_THREADS))
+                return false;
+        return true;
+    };
+    // Two pairs a thread halve the address, twiddle and LDS instructions
+    // (1040^2 FP32, 4 derivatives: 19.0 against 23.3 us), one pair halves
+    // the serial chain and wins where the grid leaves compute units idle
+    // (200^2: 6.6 against 8.2 us).  FP64 values of two pairs take all 256
+    // registers (1040^2: 44 against 40 us).
+    FftShape s;
+    s.V = elt == 4 && fits(2, 1) && blocks(2, 1) >= 2 * g.cus ? 2 : 1;
+    // Workgroups are much alike, so the launch takes the time of the compute
+    // unit with the most of them: P that leaves them evenly spread, and of
+    // two alike the larger, whose x accesses cover more of a cache line
+    // (1024^2 FP32: 15.9 us with 2 groups, 512 workgroups, 18.2 with 1;
+    // 1040^2: 24.0 with 2, 520 workgroups, 19.0 with 1).
+    s.P = 1;
+    double best = 1e30;
+    for (int P = 1; P <= 4; P *= 2) {
+        if (P > 1 && !fits(s.V, P)) break;
+        const double b = blocks(s.V, P);
+        const double t = std::ceil(b / g.cus) * g.cus / b * (P == 1 ? 1.08 : 1.0);
+        if (t <= best) { best = t; s.P = P; }
     }
-    return c;
-}
-
-inline size_t dfft_lds(int n, int P, size_t elt, int tsz)
-{
-    return (2 * (size_t)P * (n + 1) + (size_t)tsz) * 2 * elt;
-}
-
-// threads of a pstd_dfft workgroup: enough for the largest pass in one
-// round (P n / R butterflies), at most 512
-inline unsigned dfft_threads(int n, int P, int nr, uint64_t code)
-{
-    int most = 0;
-    for (int q = 0; q < nr; ++q) most = std::max(most, P * n / FFT_RADICES[(code >> (4 * q)) & 15]);
-    return (unsigned)std::min(512, std::max(64, (most + 63) / 64 * 64));
+    return s;
 }
 
 // the arguments, LDS bytes and threads of the derivatives jobs[0..nj)
 // along axis of the fields of x into d (own transforms)
 template <typename T>
-DfftArgs<T> dfft_args(const Grid &g, int axis, const T *x, T *d, const DJob *jobs, int nj, size_t &lds,
-                      unsigned &nt)
+DfftArgs<T> dfft_args(const Grid &g, int axis, const T *x, T *d, const DJob *jobs, int nj, FftShape sh,
+                      size_t &lds, unsigned &nt)
 {
     DfftArgs<T> a;
     a.x = x; a.d = d; a.N = (unsigned)g.N;
@@ -578,57 +267,75 @@ DfftArgs<T> dfft_args(const Grid &g, int axis, const T *x, T *d, const DJob *job
         a.slots |= (uint32_t)jobs[q].slot << (4 * q);
         a.fwd |= (uint32_t)(jobs[q].fwd ? 1 : 0) << q;
     }
-    a.njobs = nj;
-    const int n = axis == 0 ? g.nx2 : g.nz2, other = axis == 0 ? g.nz2 : g.nx2;
+    const FftPlan &f = g.fft[axis];
+    a.lim = axis == 0 ? g.nz2 : g.nx2;
     a.tw = (const Cx<T> *)g.tw[axis].ptr;
     a.mul_f = (const Cx<T> *)g.fmul[axis].ptr;
-    a.mul_b = a.mul_f + n;
-    a.n = n; a.nr = g.nr[axis]; a.code = g.rcode[axis]; a.tsz = tw_count(a.nr, a.code);
-    a.nx2 = g.nx2; a.nz2 = g.nz2;
-    a.P = g.P[axis];
-    a.ntiles = ((other + 1) / 2 + a.P - 1) / a.P;
+    a.mul_b = a.mul_f + f.m;
+    a.n = f.n; a.m = f.m; a.nr = f.nr; a.tsz = f.tsz;
+    auto magic = [](uint32_t v) { return v > 1 ? (uint32_t)(((1ull << 32) + v - 1) / v) : 0u; };
+    for (int q = 0; q < FFT_MAXPASS; ++q) {
+        a.radix[q] = q < f.nr ? f.R[q] : 2;
+        a.S[q] = q < f.nr ? f.S[q] : 1;
+        a.nb[q] = q < f.nr ? f.m / f.R[q] : 1;
+        a.toff[q] = q < f.nr ? f.toff[q] : 0;
+        a.mS[q] = magic(a.S[q]);
+        a.mN[q] = magic(a.nb[q]);
+    }
+    const int RL = f.R[f.nr - 1];
+    a.mL = magic(RL);
+    a.pad = RL % 2 == 0 ? 1 : 0;
+    a.P = sh.P;
+    a.lP = 0;
+    while ((1 << a.lP) < a.P) ++a.lP;
+    a.ls = fft_line(f, sh.V, sh.P, sizeof(T));
+    a.nz2 = g.nz2;
+    const int V = sh.V;
+    a.vec = g.nz2 % (2 * V) == 0 ? 2 * V : g.nz2 % 2 == 0 ? 2 : 0;
+    a.ntiles = (a.lim + 2 * V * a.P - 1) / (2 * V * a.P);
     a.nblocks = nj * a.ntiles;
-    lds = dfft_lds(n, a.P, sizeof(T), a.tsz);
-    nt = dfft_threads(n, a.P, a.nr, a.code);
+    lds = fft_lds(f, V, a.P, sizeof(T));
+    nt = (unsigned)fft_threads(f, a.P);
     return a;
 }
 
-// the derivatives jobs[0..nj) along axis of the fields of x into d
-template <typename T>
-int deriv_batch(Grid &g, int axis, const T *x, T *d, const DJob *jobs, int nj)
-{
-    if (!g.own[axis]) {
-        for (int q = 0; q < nj; ++q) {
-            int rc = deriv<T>(g, x + (size_t)jobs[q].field * g.N, axis, jobs[q].fwd, d + (size_t)jobs[q].slot * g.N);
-            if (rc != SM_OK) return rc;
-        }
-        return SM_OK;
-    }
-    size_t lds;
-    unsigned nt;
-    const DfftArgs<T> a = dfft_args<T>(g, axis, x, d, jobs, nj, lds, nt);
-    const unsigned grid = (unsigned)((a.nblocks + 7) / 8 * 8);
-    if (axis == 0) pstd_dfft<T, 0><<<grid, nt, lds, g.ctx->stream>>>(a);
-    else pstd_dfft<T, 1><<<grid, nt, lds, g.ctx->stream>>>(a);
-    return SM_OK;
-}
-
 // the derivatives xj[0..nx) along x and zj[0..nz) along z of the fields
-// of x into d: one launch when both axes use the own transforms
+// of x into d: one launch for the axes with own transforms
 template <typename T>
 int deriv_xz(Grid &g, const T *x, T *d, const DJob *xj, int nx, const DJob *zj, int nz)
 {
-    if (!(g.own[0] && g.own[1] && nx > 0 && nz > 0)) {
-        int rc = nx ? deriv_batch<T>(g, 0, x, d, xj, nx) : SM_OK;
-        if (rc == SM_OK && nz) rc = deriv_batch<T>(g, 1, x, d, zj, nz);
-        return rc;
+    const DJob *jobs[2] = {xj, zj};
+    int count[2] = {nx, nz};
+    for (int ax = 0; ax < 2; ++ax) {
+        if (g.own[ax]) continue;
+        for (int q = 0; q < count[ax]; ++q) {
+            const DJob &j = jobs[ax][q];
+            int rc = deriv<T>(g, x + (size_t)j.field * g.N, ax, j.fwd, d + (size_t)j.slot * g.N);
+            if (rc != SM_OK) return rc;
+        }
+        count[ax] = 0;
     }
-    size_t lx, lz;
-    unsigned tx, tz;
-    const DfftArgs<T> ax = dfft_args<T>(g, 0, x, d, xj, nx, lx, tx);
-    const DfftArgs<T> az = dfft_args<T>(g, 1, x, d, zj, nz, lz, tz);
-    const unsigned grid = (unsigned)((ax.nblocks + az.nblocks + 7) / 8 * 8);
-    pstd_dfft_xz<T><<<grid, std::max(tx, tz), std::max(lx, lz), g.ctx->stream>>>(ax, az);
+    if (count[0] + count[1] == 0) return SM_OK;
+    DfftArgs<T> a[2] = {};
+    size_t lds = 0;
+    unsigned nt = 64;
+    const FftShape sh = fft_shape(g, sizeof(T), count[0], count[1]);
+    for (int ax = 0; ax < 2; ++ax) {
+        if (!count[ax]) continue;
+        size_t l;
+        unsigned t;
+        a[ax] = dfft_args<T>(g, ax, x, d, jobs[ax], count[ax], sh, l, t);
+        lds = std::max(lds, l);
+        nt = std::max(nt, t);
+    }
+    const unsigned grid = (unsigned)((a[0].nblocks + 7) / 8 + (a[1].nblocks + 7) / 8) * 8;
+    if constexpr (sizeof(T) == 4) {
+        if (sh.V == 2) {
+            pstd_dfft<T, 2><<<grid, nt, lds, g.ctx->stream>>>(a[0], a[1]);
+            return SM_OK;
+        }
+    }
+    pstd_dfft<T, 1><<<grid, nt, lds, g.ctx->stream>>>(a[0], a[1]);
     return SM_OK;
 }
 
@@ -745,6 +452,23 @@ inline size_t kmul_bytes(size_t nx2, size_t nz2, size_t elt)
     return 2 * (std::max(nx2, nx2 / 2 + 1) + nz2 / 2 + 1) * 2 * elt;
 }
 
+// LDS one workgroup of transforms may take: all 160 KiB of a compute unit
+// when the runtime grants it
+inline size_t fft_lds_limit(size_t elt)
+{
+    const int want = 160 * 1024;
+    const void *k8[] = {(const void *)pstd_dfft<double, 1>}, *k4[] = {(const void *)pstd_dfft<float, 1>,
+                                                                       (const void *)pstd_dfft<float, 2>};
+    bool ok = true;
+    auto grant = [&](const void *k) {
+        ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess;
+    };
+    if (elt == 8) for (const void *k : k8) grant(k);
+    else for (const void *k : k4) grant(k);
+    (void)hipGetLastError();
+    return ok ? (size_t)want : 65536;
+}
+
 // plans, multipliers and CPML tables for an nx2 x nz2 grid with np layers;
 // own: hand-written transforms on the axes whose length allows them
 inline int init(Grid &g, sm_ctx *ctx, size_t nx2, size_t nz2, size_t np, size_t elt, double dx, double dz,
@@ -807,65 +531,37 @@ inline int init(Grid &g, sm_ctx *ctx, size_t nx2, size_t nz2, size_t np, size_t 
         for (int r = 0; r < K_NK; ++r) t.insert(t.end(), kz[r].begin(), kz[r].end());
         rc = upload_any(elt, g.tabs.ptr, t, st);
     }
-    // hand-written transforms: twiddles e^{-2 pi i k/n} and the multipliers
-    // over the whole spectrum; P pairs per workgroup within 80 KiB of LDS
-    // (two workgroups per CU)
-    int lds_max = 65536;
-    if (own) {
-        const size_t want = 81920;
-        const bool ok = elt == 8
-            ? hipFuncSetAttribute((const void *)pstd_dfft<double, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess &&
-              hipFuncSetAttribute((const void *)pstd_dfft<double, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess &&
-              hipFuncSetAttribute((const void *)pstd_dfft_xz<double>, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess
-            : hipFuncSetAttribute((const void *)pstd_dfft<float, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess &&
-              hipFuncSetAttribute((const void *)pstd_dfft<float, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess &&
-              hipFuncSetAttribute((const void *)pstd_dfft_xz<float>, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess;
-        (void)hipGetLastError();
-        if (ok) lds_max = (int)want;
-    }
+    // hand-written transforms: twiddles and the multipliers over the whole
+    // spectrum in the order of the middle pass
+    const size_t lds_limit = own ? fft_lds_limit(elt) : 0;
+    if (hipDeviceGetAttribute(&g.cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess || g.cus < 1)
+        g.cus = 256;
     for (int ax = 0; ax < 2 && rc == SM_OK && own; ++ax) {
         const size_t n = ax == 0 ? nx2 : nz2;
         const double d = ax == 0 ? dx : dz;
-        if (!fft_factor((int)n, g.nr[ax], g.rcode[ax])) continue;
-        const int tsz = tw_count(g.nr[ax], g.rcode[ax]);
-        if (dfft_lds((int)n, 1, elt, tsz) > (size_t)lds_max) continue;
-        // 4 column or row pairs per workgroup where LDS allows (adjacent
-        // x columns share cache lines; measured on 1040-point axes, FP32:
-        // 4/4 pairs 9% faster per step than 4/2, 2/2 and 1/1 slower still)
-        g.P[ax] = std::max(1, std::min(4, (int)(lds_max / dfft_lds((int)n, 1, elt, tsz))));
-        while (g.P[ax] > 1 && dfft_lds((int)n, g.P[ax], elt, tsz) > (size_t)lds_max) --g.P[ax];
-        std::vector<double> tw, fm;
+        FftPlan &f = g.fft[ax];
+        if (!fft_plan((int)n, f) || fft_lds(f, 1, 1, elt) > lds_limit || fft_threads(f, 1) > FFT_THREADS) continue;
         const double two_pi = 8.0 * std::atan(1.0);
-        // per pass: e^{-2 pi i k t / (Ns R)} at (t - 1) Ns + k, then the
-        // R-th roots of unity
-        for (int q = 0, Ns = 1; q < g.nr[ax]; ++q) {
-            const int R = FFT_RADICES[(g.rcode[ax] >> (4 * q)) & 15];
-            for (int t = 1; t < R; ++t)
-                for (int k = 0; k < Ns; ++k) {
-                    const double th = two_pi * (double)k * t / ((double)Ns * R);
-                    tw.push_back(std::cos(th)); tw.push_back(-std::sin(th));
-                }
-            for (int m = 0; m < R; ++m) {
-                const double th = two_pi * (double)m / R;
-                tw.push_back(std::cos(th)); tw.push_back(-std::sin(th));
-            }
-            Ns *= R;
-        }
+        std::vector<double> fm;
         for (double sgn : {1.0, -1.0}) {
             const double dn = two_pi / (d * n * n);
             auto h = [&](size_t m, double &re, double &im) {
                 const double k = m * dn, ph = sgn * 0.5 * k * d * n;
                 re = -k * std::sin(ph); im = k * std::cos(ph);
             };
-            for (size_t m = 0; m < n; ++m) {
-                double re, im;
-                if (2 * m < n) h(m, re, im);
-                else if (2 * m == n) { h(m, re, im); im = 0.0; }
-                else { h(n - m, re, im); im = -im; }
-                fm.push_back(re); fm.push_back(im);
-            }
+            const int RL = f.R[f.nr - 1], nb = f.m / RL;
+            for (int t = 0; t < RL; ++t)
+                for (int b = 0; b < nb; ++b) {
+                    const size_t m = (size_t)fft_freq(f, b, t);
+                    double re, im;
+                    if (2 * m < n) h(m, re, im);
+                    else if (2 * m == n) { h(m, re, im); im = 0.0; }
+                    else { h(n - m, re, im); im = -im; }
+                    fm.push_back(re); fm.push_back(im);
+                }
         }
-        rc = dalloc(g.tw[ax], tw.size() * elt);
+        const std::vector<double> tw = fft_twiddles(f);
+        rc = dalloc(g.tw[ax], std::max<size_t>(tw.size(), 2) * elt);
         if (rc == SM_OK) rc = dalloc(g.fmul[ax], fm.size() * elt);
         if (rc == SM_OK) rc = upload_any(elt, g.tw[ax].ptr, tw, st);
         if (rc == SM_OK) rc = upload_any(elt, g.fmul[ax].ptr, fm, st);
@@ -895,10 +591,13 @@ inline int init(Grid &g, sm_ctx *ctx, size_t nx2, size_t nz2, size_t np, size_t 
 // device bytes of the machinery
 inline size_t grid_bytes(size_t nx2, size_t nz2, size_t np, size_t elt)
 {
-    // per axis: twiddles and roots (n - 1 + the sum of the radices) and two
-    // multiplier tables of n
-    return spec_bytes(nx2, nz2, elt) + kmul_bytes(nx2, nz2, elt) + table_bytes(np, elt) +
-           (3 * (nx2 + nz2) + 2 * 16 * FFT_MAXPASS) * 2 * elt;
+    // per axis: twiddles and two multiplier tables
+    size_t own = 0;
+    for (size_t n : {nx2, nz2}) {
+        FftPlan f;
+        if (fft_plan((int)n, f)) own += ((size_t)std::max(f.tsz, 1) + 2 * (size_t)f.m) * 2 * elt;
+    }
+    return spec_bytes(nx2, nz2, elt) + kmul_bytes(nx2, nz2, elt) + table_bytes(np, elt) + own;
 }
 
 inline size_t grid_device_bytes(const Grid &g)
