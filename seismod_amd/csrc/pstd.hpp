@@ -18,10 +18,11 @@
 //   z (unit stride): real-to-complex and complex-to-real transforms.
 // Results equal the real-transform derivatives to rounding.
 //
-// When an axis length factors into 2, 3, 5, 7, 11 and 13, its derivatives
-// skip hipFFT: one pstd_dfft launch (pstd_fft.hpp) takes every derivative of
-// a stage along both axes, with one read and one write per value instead of
-// six (forward transform, multiplier pass, inverse transform).
+// Axes whose transforms fit a workgroup's LDS skip hipFFT: one pstd_dfft
+// launch (pstd_fft.hpp) takes every derivative of a stage along both axes,
+// with one read and one write per value instead of six (forward transform,
+// multiplier pass, inverse transform).  hipFFT remains for longer axes and
+// on request (SM_PSTD_HIPFFT).
 //
 // CPML (pml.c:1959-2106): per stage (fp1, fp23, fp4) and axis the rows b,
 // c at nodes, bh, ch at inner half nodes, bH, cH at outer half nodes; the
@@ -329,13 +330,17 @@ int deriv_xz(Grid &g, const T *x, T *d, const DJob *xj, int nx, const DJob *zj, 
         nt = std::max(nt, t);
     }
     const unsigned grid = (unsigned)((a[0].nblocks + 7) / 8 + (a[1].nblocks + 7) / 8) * 8;
+    const bool pad = (count[0] && g.fft[0].m != g.fft[0].n) || (count[1] && g.fft[1].m != g.fft[1].n);
+    hipStream_t st = g.ctx->stream;
     if constexpr (sizeof(T) == 4) {
         if (sh.V == 2) {
-            pstd_dfft<T, 2><<<grid, nt, lds, g.ctx->stream>>>(a[0], a[1]);
+            if (pad) pstd_dfft<T, 2, true><<<grid, nt, lds, st>>>(a[0], a[1]);
+            else pstd_dfft<T, 2, false><<<grid, nt, lds, st>>>(a[0], a[1]);
             return SM_OK;
         }
     }
-    pstd_dfft<T, 1><<<grid, nt, lds, g.ctx->stream>>>(a[0], a[1]);
+    if (pad) pstd_dfft<T, 1, true><<<grid, nt, lds, st>>>(a[0], a[1]);
+    else pstd_dfft<T, 1, false><<<grid, nt, lds, st>>>(a[0], a[1]);
     return SM_OK;
 }
 
@@ -457,8 +462,9 @@ inline size_t kmul_bytes(size_t nx2, size_t nz2, size_t elt)
 inline size_t fft_lds_limit(size_t elt)
 {
     const int want = 160 * 1024;
-    const void *k8[] = {(const void *)pstd_dfft<double, 1>}, *k4[] = {(const void *)pstd_dfft<float, 1>,
-                                                                       (const void *)pstd_dfft<float, 2>};
+    const void *k8[] = {(const void *)pstd_dfft<double, 1, false>, (const void *)pstd_dfft<double, 1, true>};
+    const void *k4[] = {(const void *)pstd_dfft<float, 1, false>, (const void *)pstd_dfft<float, 1, true>,
+                        (const void *)pstd_dfft<float, 2, false>, (const void *)pstd_dfft<float, 2, true>};
     bool ok = true;
     auto grant = [&](const void *k) {
         ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess;
@@ -540,24 +546,15 @@ inline int init(Grid &g, sm_ctx *ctx, size_t nx2, size_t nz2, size_t np, size_t 
         const size_t n = ax == 0 ? nx2 : nz2;
         const double d = ax == 0 ? dx : dz;
         FftPlan &f = g.fft[ax];
-        if (!fft_plan((int)n, f) || fft_lds(f, 1, 1, elt) > lds_limit || fft_threads(f, 1) > FFT_THREADS) continue;
-        const double two_pi = 8.0 * std::atan(1.0);
+        if (!fft_plan((int)n, f) || fft_lds(f, 1, 1, elt) > lds_limit) continue;
         std::vector<double> fm;
         for (double sgn : {1.0, -1.0}) {
-            const double dn = two_pi / (d * n * n);
-            auto h = [&](size_t m, double &re, double &im) {
-                const double k = m * dn, ph = sgn * 0.5 * k * d * n;
-                re = -k * std::sin(ph); im = k * std::cos(ph);
-            };
+            const std::vector<double> h = fft_spectrum(f, d, sgn);
             const int RL = f.R[f.nr - 1], nb = f.m / RL;
             for (int t = 0; t < RL; ++t)
                 for (int b = 0; b < nb; ++b) {
-                    const size_t m = (size_t)fft_freq(f, b, t);
-                    double re, im;
-                    if (2 * m < n) h(m, re, im);
-                    else if (2 * m == n) { h(m, re, im); im = 0.0; }
-                    else { h(n - m, re, im); im = -im; }
-                    fm.push_back(re); fm.push_back(im);
+                    const size_t k = (size_t)fft_freq(f, b, t);
+                    fm.push_back(h[2 * k]); fm.push_back(h[2 * k + 1]);
                 }
         }
         const std::vector<double> tw = fft_twiddles(f);

@@ -295,21 +295,124 @@ inline bool fft_radices(int m, FftPlan &p)
     return true;
 }
 
-// plan of the derivative of n points; false when no hand-written transform
-// takes this length
-inline bool fft_plan(int n, FftPlan &p)
+inline void fft_layout(FftPlan &p)
 {
-    p = FftPlan();
-    if (n < 4 || !fft_radices(n, p)) return false;
-    p.n = p.m = n;
     int B = p.m;
+    p.tsz = 0;
     for (int q = 0; q < p.nr; ++q) {
         p.S[q] = B / p.R[q];
         p.toff[q] = p.tsz;
         if (p.S[q] > 1) p.tsz += (p.R[q] - 1) * p.S[q];
         B = p.S[q];
     }
-    return true;
+}
+
+constexpr int FFT_THREADS = 512;    // largest workgroup: 256 registers a thread
+// threads of a workgroup: every pass takes its butterflies in one round
+inline int fft_threads(const FftPlan &p, int P)
+{
+    int most = 0;
+    for (int q = 0; q < p.nr; ++q) most = std::max(most, P * (p.m / p.R[q]));
+    return (most + 63) / 64 * 64;
+}
+
+// plan of the derivative of n points; false when no hand-written transform
+// takes this length.  The derivative is a circular convolution with a real
+// kernel of n points, so a length with other factors runs as a linear one:
+// lines padded with zeros to any m >= 2 n - 1 that the radices make, and the
+// kernel's spectrum over m points as the multiplier: twice the work of a
+// length that the radices make (1039^2 against 1040^2, 8 FP32 derivatives:
+// 77.6 and 36.2 us), a quarter of hipFFT's chirp transforms and their copy
+// passes (469 x 363, FP64, a P-SV stage: 45 against 230 us).
+inline bool fft_plan(int n, FftPlan &p)
+{
+    p = FftPlan();
+    if (n < 2) return false;
+    if (fft_radices(n, p)) {
+        p.m = n;
+    } else {
+        FftPlan best;
+        double cost = 1e30;
+        for (int m = 2 * n - 1; m <= 2 * n + n / 4 + 16; ++m) {
+            FftPlan f;
+            if (!fft_radices(m, f) || f.cost * m >= cost) continue;
+            f.m = m;
+            if (fft_threads(f, 1) > FFT_THREADS) continue;
+            cost = f.cost * m;
+            best = f;
+        }
+        if (best.nr == 0) return false;
+        p = best;
+    }
+    p.n = n;
+    fft_layout(p);
+    return fft_threads(p, 1) <= FFT_THREADS;
+}
+
+// whole-spectrum multiplier of the forward (sgn 1) or backward (-1)
+// derivative of n points of spacing d, 1 / n of the inverse included: the
+// Nyquist bin real, as a complex-to-real inverse takes it
+inline void fft_multiplier(int n, double d, double sgn, int k, double &re, double &im)
+{
+    const double two_pi = 8.0 * std::atan(1.0);
+    const int q = 2 * k <= n ? k : n - k;
+    const double w = q * (two_pi / (d * n * n)), ph = sgn * 0.5 * w * d * n;
+    re = -w * std::sin(ph);
+    im = 2 * k == n ? 0.0 : (2 * k < n ? 1.0 : -1.0) * w * std::cos(ph);
+}
+
+// the multiplier over the m points of plan p, in natural order
+inline std::vector<double> fft_spectrum(const FftPlan &p, double d, double sgn)
+{
+    const int n = p.n, m = p.m;
+    std::vector<double> out(2 * (size_t)m);
+    if (m == n) {
+        for (int k = 0; k < n; ++k) fft_multiplier(n, d, sgn, k, out[2 * k], out[2 * k + 1]);
+        return out;
+    }
+    // (sums in extended precision: their rounding would be the largest error
+    // of an FP64 derivative)
+    typedef long double L;
+    const L two_pi = 8.0L * std::atan(1.0L);
+    auto roots = [&](int len) {
+        std::vector<L> w(2 * (size_t)len);
+        for (int q = 0; q < len; ++q) {
+            w[2 * q] = std::cos(two_pi * q / len);
+            w[2 * q + 1] = std::sin(two_pi * q / len);
+        }
+        return w;
+    };
+    // kernel c[j] = sum_k H(k) e^{2 pi i j k / n}; H(n - k) = conj H(k)
+    std::vector<L> c(n, 0.0L), w = roots(n);
+    std::vector<L> h(n + 2);
+    for (int k = 0; 2 * k <= n; ++k) {
+        const L wk = k * (two_pi / ((L)d * n * n)), ph = sgn * 0.5L * wk * d * n;
+        h[2 * k] = -wk * std::sin(ph);
+        h[2 * k + 1] = 2 * k == n ? 0.0L : wk * std::cos(ph);
+    }
+    for (int j = 0; j < n; ++j)
+        for (int k = 1; 2 * k <= n; ++k) {
+            const size_t q = (size_t)((int64_t)j * k % n);
+            c[j] += (2 * k == n ? 1.0L : 2.0L) * (h[2 * k] * w[2 * q] - h[2 * k + 1] * w[2 * q + 1]);
+        }
+    // its spectrum: kernel positions -(n - 1) .. n - 1 of the m points
+    w = roots(m);
+    for (int k = 0; 2 * k <= m; ++k) {
+        L re = 0.0L, im = 0.0L;
+        size_t q = (size_t)(((int64_t)(1 - n) * k) % m + m) % m;
+        for (int j = 1 - n; j < n; ++j) {
+            const L v = c[j < 0 ? j + n : j];
+            re += v * w[2 * q];
+            im -= v * w[2 * q + 1];
+            q += k;
+            if (q >= (size_t)m) q -= m;
+        }
+        const size_t r = (size_t)((m - k) % m);
+        out[2 * k] = out[2 * r] = (double)(re / m);
+        out[2 * k + 1] = (double)(im / m);
+        if (r != (size_t)k) out[2 * r + 1] = (double)(-im / m);
+    }
+    return out;
 }
 
 // twiddles of every pass, (re, im) pairs
@@ -367,7 +470,6 @@ __device__ __forceinline__ uint32_t divm(uint32_t l, uint32_t m) { return m ? __
 
 // a group of V pairs at one position: one thread takes all of them, so that
 // addresses, twiddles, multipliers and roots serve V transforms
-constexpr int FFT_THREADS = 512;    // largest workgroup: 256 registers a thread
 template <typename T, int V>
 struct __align__(V * 2 * sizeof(T) < 16 ? V * 2 * sizeof(T) : 16) Elem {
     Cx<T> c[V];
@@ -396,11 +498,13 @@ __device__ __forceinline__ void outer_item(const DfftArgs<T> &a, uint32_t l, uin
 }
 
 // v[g][t] <- elements j + t S of group g's pair of lines
-template <typename T, int V, int R, int AX>
+template <typename T, int V, int R, int AX, bool PAD>
 __device__ __forceinline__ void load_lines(const DfftArgs<T> &a, const FftIO<T, V> &io, int p, uint32_t j,
                                            Cx<T> (&v)[V][R])
 {
     const uint32_t S = a.S[0];
+    // elements from n on (a padded line) are 0 and have no derivative
+    auto in = [&](int t) { return !PAD || j + t * S < (uint32_t)a.n; };
     const int r0 = io.r0 + 2 * V * p;
     if (AX == 0) {
         const T *f = io.f + (size_t)j * a.nz2 + r0;
@@ -408,6 +512,7 @@ __device__ __forceinline__ void load_lines(const DfftArgs<T> &a, const FftIO<T, 
         if (a.vec == 2 * V && r0 + 2 * V <= a.lim) {
 #pragma unroll
             for (int t = 0; t < R; ++t) {
+                if (!in(t)) continue;
                 const Elem<T, V> e = *(const Elem<T, V> *)(f + t * st);
 #pragma unroll
                 for (int g = 0; g < V; ++g) v[g][t] = e.c[g];
@@ -420,16 +525,16 @@ __device__ __forceinline__ void load_lines(const DfftArgs<T> &a, const FftIO<T, 
             if (a.vec) {
                 if (r < a.lim) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) v[g][t] = *(const Cx<T> *)(f + 2 * g + t * st);
+                    for (int t = 0; t < R; ++t) if (in(t)) v[g][t] = *(const Cx<T> *)(f + 2 * g + t * st);
                 }
             } else {
                 if (r < a.lim) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) v[g][t].re = f[2 * g + t * st];
+                    for (int t = 0; t < R; ++t) if (in(t)) v[g][t].re = f[2 * g + t * st];
                 }
                 if (r + 1 < a.lim) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) v[g][t].im = f[2 * g + t * st + 1];
+                    for (int t = 0; t < R; ++t) if (in(t)) v[g][t].im = f[2 * g + t * st + 1];
                 }
             }
         }
@@ -440,22 +545,24 @@ __device__ __forceinline__ void load_lines(const DfftArgs<T> &a, const FftIO<T, 
             const T *f = io.f + (size_t)r * a.nz2 + j;
             if (r < a.lim) {
 #pragma unroll
-                for (int t = 0; t < R; ++t) v[g][t].re = f[t * S];
+                for (int t = 0; t < R; ++t) if (in(t)) v[g][t].re = f[t * S];
             }
             if (r + 1 < a.lim) {
 #pragma unroll
-                for (int t = 0; t < R; ++t) v[g][t].im = f[a.nz2 + t * S];
+                for (int t = 0; t < R; ++t) if (in(t)) v[g][t].im = f[a.nz2 + t * S];
             }
         }
     }
 }
 
 // the conjugates of v[g][t] -> elements j + t S of the derivatives
-template <typename T, int V, int R, int AX>
+template <typename T, int V, int R, int AX, bool PAD>
 __device__ __forceinline__ void store_lines(const DfftArgs<T> &a, const FftIO<T, V> &io, int p, uint32_t j,
                                             const Cx<T> (&v)[V][R])
 {
     const uint32_t S = a.S[0];
+    // elements from n on (a padded line) are 0 and have no derivative
+    auto in = [&](int t) { return !PAD || j + t * S < (uint32_t)a.n; };
     const int r0 = io.r0 + 2 * V * p;
     if (AX == 0) {
         T *o = io.out + (size_t)j * a.nz2 + r0;
@@ -463,6 +570,7 @@ __device__ __forceinline__ void store_lines(const DfftArgs<T> &a, const FftIO<T,
         if (a.vec == 2 * V && r0 + 2 * V <= a.lim) {
 #pragma unroll
             for (int t = 0; t < R; ++t) {
+                if (!in(t)) continue;
                 Elem<T, V> e;
 #pragma unroll
                 for (int g = 0; g < V; ++g) e.c[g] = {v[g][t].re, -v[g][t].im};
@@ -476,16 +584,16 @@ __device__ __forceinline__ void store_lines(const DfftArgs<T> &a, const FftIO<T,
             if (a.vec) {
                 if (r < a.lim) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) *(Cx<T> *)(o + 2 * g + t * st) = {v[g][t].re, -v[g][t].im};
+                    for (int t = 0; t < R; ++t) if (in(t)) *(Cx<T> *)(o + 2 * g + t * st) = {v[g][t].re, -v[g][t].im};
                 }
             } else {
                 if (r < a.lim) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) o[2 * g + t * st] = v[g][t].re;
+                    for (int t = 0; t < R; ++t) if (in(t)) o[2 * g + t * st] = v[g][t].re;
                 }
                 if (r + 1 < a.lim) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) o[2 * g + t * st + 1] = -v[g][t].im;
+                    for (int t = 0; t < R; ++t) if (in(t)) o[2 * g + t * st + 1] = -v[g][t].im;
                 }
             }
         }
@@ -496,11 +604,11 @@ __device__ __forceinline__ void store_lines(const DfftArgs<T> &a, const FftIO<T,
             T *o = io.out + (size_t)r * a.nz2 + j;
             if (r < a.lim) {
 #pragma unroll
-                for (int t = 0; t < R; ++t) o[t * S] = v[g][t].re;
+                for (int t = 0; t < R; ++t) if (in(t)) o[t * S] = v[g][t].re;
             }
             if (r + 1 < a.lim) {
 #pragma unroll
-                for (int t = 0; t < R; ++t) o[a.nz2 + t * S] = -v[g][t].im;
+                for (int t = 0; t < R; ++t) if (in(t)) o[a.nz2 + t * S] = -v[g][t].im;
             }
         }
     }
@@ -545,7 +653,7 @@ __device__ __forceinline__ void dft_group(Cx<T> (&v)[V][R])
 }
 
 // first pass: global memory -> LDS
-template <typename T, int V, int R, int AX>
+template <typename T, int V, int R, int AX, bool PAD>
 __device__ __forceinline__ void pass_first(const DfftArgs<T> &a, const FftIO<T, V> &io)
 {
     const uint32_t S = a.S[0], items = a.nb[0] << a.lP;
@@ -559,7 +667,7 @@ __device__ __forceinline__ void pass_first(const DfftArgs<T> &a, const FftIO<T, 
         for (int t = 0; t < R; ++t) v[g][t] = {T(0), T(0)};
     if (l < items) {
         outer_item<T, AX>(a, l, p, j);
-        load_lines<T, V, R, AX>(a, io, (int)p, j, v);
+        load_lines<T, V, R, AX, PAD>(a, io, (int)p, j, v);
     }
     // the twiddle table, while the lines are on their way
     for (int q = threadIdx.x; q < a.tsz; q += blockDim.x) io.tw[q] = a.tw[q];
@@ -620,7 +728,7 @@ __device__ __forceinline__ void pass_mid(const DfftArgs<T> &a, const FftIO<T, V>
 }
 
 // last pass: LDS -> global memory
-template <typename T, int V, int R, int AX>
+template <typename T, int V, int R, int AX, bool PAD>
 __device__ __forceinline__ void pass_last(const DfftArgs<T> &a, const FftIO<T, V> &io)
 {
     const uint32_t S = a.S[0], items = a.nb[0] << a.lP;
@@ -633,7 +741,7 @@ __device__ __forceinline__ void pass_last(const DfftArgs<T> &a, const FftIO<T, V
         lds_load<T, V, R>(io.A + p * a.ls + lds_at(a, j), lst, v);
         twiddle<T, V, R>(io.tw + j, S, v);
         dft_group<T, V, R>(v);
-        store_lines<T, V, R, AX>(a, io, (int)p, j, v);
+        store_lines<T, V, R, AX, PAD>(a, io, (int)p, j, v);
     }
 }
 
@@ -658,7 +766,7 @@ __device__ __forceinline__ void pass_last(const DfftArgs<T> &a, const FftIO<T, V
 // the derivative of the lines of tile b: AX 1 z (unit stride, row pairs
 // r, r + 1), AX 0 x (stride nz2, column pairs c, c + 1); a missing partner
 // reads as 0 and is not written
-template <typename T, int V, int AX>
+template <typename T, int V, int AX, bool PAD>
 __device__ __forceinline__ void dfft_body(const DfftArgs<T> &a, int b)
 {
     const int jb = b / a.ntiles, tile = b - jb * a.ntiles;
@@ -669,7 +777,7 @@ __device__ __forceinline__ void dfft_body(const DfftArgs<T> &a, int b)
     io.A = (Elem<T, V> *)pstd_lds;
     io.tw = (Cx<T> *)(io.A + a.P * a.ls);
     const Cx<T> *mul = ((a.fwd >> jb) & 1) ? a.mul_f : a.mul_b;
-    PSTD_RADIX(a.radix[0], (pass_first<T, V, R, AX>(a, io)))
+    PSTD_RADIX(a.radix[0], (pass_first<T, V, R, AX, PAD>(a, io)))
     __syncthreads();
     // the inner passes forward, the middle, the inner passes back
     const int inner = a.nr - 2;
@@ -682,23 +790,23 @@ __device__ __forceinline__ void dfft_body(const DfftArgs<T> &a, int b)
         }
         __syncthreads();
     }
-    PSTD_RADIX(a.radix[0], (pass_last<T, V, R, AX>(a, io)))
+    PSTD_RADIX(a.radix[0], (pass_last<T, V, R, AX, PAD>(a, io)))
 }
 
 // the derivatives of a stage along x (ax) and z (az) in one grid (either may
-// have none).  Every XCD takes a range of consecutive x tiles (adjacent
+// have none); PAD: a line is shorter than its transform.  Every XCD takes a range of consecutive x tiles (adjacent
 // columns share cache lines) and then a range of z tiles: the x tiles move
 // more cache lines and take longer, so giving half of the XCDs only x tiles
 // would leave the others waiting.
-template <typename T, int V>
+template <typename T, int V, bool PAD>
 __global__ __launch_bounds__(FFT_THREADS) void pstd_dfft(const DfftArgs<T> ax, const DfftArgs<T> az)
 {
     const int px = (ax.nblocks + 7) / 8, pz = (az.nblocks + 7) / 8;
     const int xcd = blockIdx.x % 8, i = blockIdx.x / 8;
     if (i < px) {
-        if (xcd * px + i < ax.nblocks) dfft_body<T, V, 0>(ax, xcd * px + i);
+        if (xcd * px + i < ax.nblocks) dfft_body<T, V, 0, PAD>(ax, xcd * px + i);
     } else {
-        if (xcd * pz + i - px < az.nblocks) dfft_body<T, V, 1>(az, xcd * pz + i - px);
+        if (xcd * pz + i - px < az.nblocks) dfft_body<T, V, 1, PAD>(az, xcd * pz + i - px);
     }
 }
 
@@ -712,13 +820,6 @@ inline int fft_line(const FftPlan &p, int V, int P, size_t elt)
     const int want = row / std::min(P, row);
     while (ls % row != want % row) ++ls;
     return ls;
-}
-// threads of a workgroup: every pass takes its butterflies in one round
-inline int fft_threads(const FftPlan &p, int P)
-{
-    int most = 0;
-    for (int q = 0; q < p.nr; ++q) most = std::max(most, P * (p.m / p.R[q]));
-    return (most + 63) / 64 * 64;
 }
 inline size_t fft_lds(const FftPlan &p, int V, int P, size_t elt)
 {

@@ -1,6 +1,6 @@
 """Spectral derivatives over axis lengths where a transform plan can go wrong:
 every radix from 2 to 16 in the first, inner and middle pass, two to four
-passes, odd numbers of lines (a pair without a partner), row pitches that do
+passes, lengths with other factors, odd numbers of lines (a pair without a partner), row pitches that do
 and do not allow vector accesses, grids with one and with two pairs a thread.
 
 A few steps of the SH solver without layers against its numpy oracle; the
@@ -24,7 +24,9 @@ pytestmark = pytest.mark.gpu
 # (nx, nz): two passes at the small end, three and four passes
 SIZES = [(4, 6), (9, 4), (10, 15), (21, 22), (26, 35), (48, 39), (49, 64), (99, 60), (121, 96), (117, 130),
          (143, 154), (165, 168), (196, 210), (225, 256), (343, 36), (14, 1001), (1029, 10), (2048, 9), (12, 2197),
-         (3003, 8), (6, 4096), (300, 308)]
+         (3003, 8), (6, 4096), (300, 308),
+         # other factors: padded lines (2 to 5 points, primes, a prime squared, odd and even)
+         (2, 3), (3, 5), (17, 7), (13, 11), (34, 33), (289, 38), (363, 469), (1021, 6), (5, 2039), (204, 418)]
 
 
 def run(ctx, nx, nz, storage):
@@ -59,6 +61,7 @@ def test_derivatives_of_every_length(ctx, size, storage):
     eps = 2.0 ** -52 if storage == "f64" else 2.0 ** -23
     tol = 100 * eps * math.log2(max(size))
     for k in range(3):
-        e = float(np.linalg.norm(got[k] - want[k]) / np.linalg.norm(want[k]))
+        # a grid of two rows has no interior node: v_y stays 0
+        e = float(np.linalg.norm(got[k] - want[k]) / (np.linalg.norm(want[k]) or 1.0))
         note("pstd_lengths", size=f"{size[0]}x{size[1]}", storage=storage, field=k, error=e, tol=tol)
-        assert np.abs(want[k]).max() > 0 and e < tol, (k, e, tol)
+        assert e < tol and (np.abs(want[k]).max() > 0 or min(size) < 3), (k, e, tol)
