@@ -295,12 +295,15 @@ int sm_e2d_device_bytes(const sm_e2d *s, size_t *bytes);
  * below 2 GiB (about 4730^2 padded cells) */
 size_t sm_e2d_bytes_needed(const sm_e2d_params *p, size_t nrec, size_t max_steps);
 
-/* Launch shape of the fused FP32 step (no counterpart in the reference):
- * x rows each wavefront marches over, and steps per captured hipGraph
- * (0 or 1: plain launches).  Results do not depend on either. */
+/* Launch shape of the fused FP32 step where a launch takes one step (runs of
+ * one step, grids above about 4230^2 padded cells, the allocation-free
+ * batches; longer runs advance several steps per launch and choose their
+ * own shape; no counterpart in the reference): x rows each wavefront marches
+ * over, and steps per captured hipGraph (0 or 1: plain launches).  Results
+ * do not depend on either. */
 int sm_e2d_set_launch(sm_e2d *s, int rows_per_chunk, int graph_steps);
 int sm_e2d_get_launch(const sm_e2d *s, int *rows_per_chunk, int *graph_steps);
-/* Kernel form of the fused FP32 step (no counterpart in the reference):
+/* Kernel form of the one-step launch (no counterpart in the reference):
  * SM_E2D_ROWS, each lane loads the rows of the next x row itself;
  * SM_E2D_STAGED, the rows every step needs arrive as 16-byte chunk loads
  * through LDS.  Results are identical. */
@@ -308,15 +311,15 @@ int sm_e2d_get_launch(const sm_e2d *s, int *rows_per_chunk, int *graph_steps);
 #define SM_E2D_STAGED 1
 int sm_e2d_set_variant(sm_e2d *s, int variant);
 int sm_e2d_get_variant(const sm_e2d *s, int *variant);
-/* HIP-event timing of every sm_e2d_run (no counterpart in the reference) */
+/* HIP-event timing of every sm_e2d_run; launches counts time steps (no
+ * counterpart in the reference) */
 int sm_e2d_set_timing(sm_e2d *s, int on);
 int sm_e2d_get_timing(const sm_e2d *s, double *ms_total, size_t *launches);
 
 /* ------------------------------------------------------------------ */
 /* Batches of independent 2D shots (no counterpart in the reference,   */
-/* which runs one shot per process).  One launch per time step advances */
-/* every shot that still has steps to run; long stretches are replayed  */
-/* from captured hipGraphs.  Each shot's results are those of running   */
+/* which runs one shot per process).  One launch advances every shot      */
+/* that still has steps to run, by several steps at a time.  Each shot's results are those of running   */
 /* it alone with sm_e2d_run.                                            */
 /* ------------------------------------------------------------------ */
 typedef struct sm_e2d_batch sm_e2d_batch;

@@ -163,8 +163,8 @@ using namespace sm;
 //  - reference-order kernels (FP64, or FP32 with SM_E2D_NAIVE): fields = 5
 //    totals + 10 split arrays, mat = b, bm, la, l2m, mu, damp = (c1, c2)
 //    pairs, src/rcv as int64 records;
-//  - fused FP32 kernel (default for FP32): fields = two parity buffers of
-//    E2_NSTATE arrays + E2_NSPLIT stress split arrays, mat = the five
+//  - fused FP32 kernels (default for FP32): fields = two buffers of
+//    E2_NSTATE arrays + one or two of E2_NSPLIT stress split arrays, mat = the five
 //    coefficients times dt/h, damp = (A, B) pairs, src/rcv as int4 records
 //    sorted by padded cell.
 struct sm_e2d {
@@ -180,6 +180,9 @@ struct sm_e2d {
     size_t step = 0, nsrc = 0, nrec = 0, max_steps = 0, rcv_step0 = 0;
     int chunk = 8, graph_steps = 32;
     int variant = SM_E2D_ROWS;
+    // fused: the state buffer and stress split buffer that hold step `step`
+    int cur = 0, scur = 0;
+    bool tiles = false;     // a second split buffer: several steps per launch possible
     sm::E2dRunner *runner = nullptr;
 };
 
@@ -279,9 +282,14 @@ E2dShot e2d_shot(sm_e2d *s, size_t nsteps)
     d.rmax = (int)s->max_steps;
     d.N = (unsigned)s->N;
     float *f = (float *)s->fields.ptr;
-    d.st[0] = f;
-    d.st[1] = f + E2_NSTATE * s->N;
-    d.ss = f + 2 * E2_NSTATE * s->N;
+    for (int h = 0; h < 2; ++h) {
+        float *st = f + (size_t)((s->cur + h) & 1) * E2_NSTATE * s->N;
+        d.st[(s->step + h) & 1] = st;
+        d.tst[h] = st;
+        d.tss[h] = s->tiles ? f + (2 * E2_NSTATE + (size_t)((s->scur + h) & 1) * E2_NSPLIT) * s->N : nullptr;
+    }
+    d.base = f;
+    d.ss = f + (2 * E2_NSTATE + (size_t)s->scur * E2_NSPLIT) * s->N;
     d.mat = (const float *)s->mat.ptr;
     d.dmp = (const float *)s->damp.ptr;
     d.src = (const int4 *)s->src.ptr;
@@ -291,6 +299,16 @@ E2dShot e2d_shot(sm_e2d *s, size_t nsteps)
     d.rrow = s->rcv.ptr ? (const int *)((const int4 *)s->rcv.ptr + s->nrec) : nullptr;
     d.trace = (float *)s->trace.ptr;
     return d;
+}
+
+// the solver's buffers after a run of nsteps in the runner's last form
+static void e2d_advance(sm_e2d *s, const E2dRunner &r, size_t nsteps)
+{
+    const size_t k = r.tile().steps;
+    const int flips = (int)((k ? (nsteps + k - 1) / k : nsteps) & 1);
+    s->cur ^= flips;
+    if (k) s->scur ^= flips;
+    s->step += nsteps;
 }
 
 int e2d_check_steps(const sm_e2d *s, size_t nsteps)
@@ -312,7 +330,7 @@ int run_fused(sm_e2d *s, size_t nsteps)
     s->runner->staged = s->variant == SM_E2D_STAGED;
     rc = s->runner->run(one, s->ctx->stream, s->graph_steps);
     if (rc != SM_OK) return rc;
-    s->step += nsteps;
+    e2d_advance(s, *s->runner, nsteps);
     return SM_OK;
 }
 
@@ -333,6 +351,7 @@ int zero_state(sm_e2d *s)
     if (s->trace.ptr) SM_HIP(hipMemsetAsync(s->trace.ptr, 0, s->trace.bytes, st));
     SM_HIP(hipStreamSynchronize(st));
     s->step = 0;
+    s->cur = s->scur = 0;
     s->rcv_step0 = 0;
     return SM_OK;
 }
@@ -362,6 +381,12 @@ static bool e2d_fused_fits(size_t N)
     return (2 * E2_NSTATE + E2_NSPLIT) * N * 4 < (1ull << 31);
 }
 
+// floats of the fused solver's state: a second split buffer, for several
+// steps per launch, as long as the whole stays below the same bound (24
+// bytes more per cell; larger grids run a launch a step as before)
+static bool e2d_tiles(size_t N) { return (2 * E2_NSTATE + 2 * E2_NSPLIT) * N * 4 < (1ull << 31); }
+static size_t e2d_state_floats(size_t N) { return (2 * E2_NSTATE + (e2d_tiles(N) ? 2 : 1) * E2_NSPLIT) * N; }
+
 size_t sm_e2d_bytes_needed(const sm_e2d_params *p, size_t nrec, size_t max_steps)
 {
     if (!p) return 0;
@@ -369,7 +394,7 @@ size_t sm_e2d_bytes_needed(const sm_e2d_params *p, size_t nrec, size_t max_steps
     const size_t NX = p->nx + 2 * p->npml, NZ = p->nz + 2 * p->npml, N = NX * NZ;
     if (p->storage == SM_STORE_F32 && !(p->flags & SM_E2D_NAIVE)) {
         if (!e2d_fused_fits(N)) return 0;   // sm_e2d_create refuses the grid
-        return 4 * ((2 * E2_NSTATE + E2_NSPLIT + E2_NMAT) * N + 4 * (NX + NZ) + nrec * max_steps) +
+        return 4 * (e2d_state_floats(N) + E2_NMAT * N + 4 * (NX + NZ) + nrec * max_steps) +
                16 * nrec + 4096;
     }
     return e * (20 * N + 4 * (NX + NZ) + nrec * max_steps) + 16 * nrec;
@@ -531,7 +556,8 @@ int sm_e2d_create(sm_ctx *ctx, const sm_e2d_params *pp, const double *vp, const 
         SM_CHECK(e2d_fused_fits(N), SM_ERR_ARG,
                  "sm_e2d_create: padded grid %zux%zu too large for the fused FP32 kernel "
                  "(state and split fields must stay below 2 GiB; use SM_E2D_NAIVE or FP64)", NX, NZ);
-        rc = dalloc(s->fields, (2 * E2_NSTATE + E2_NSPLIT) * N * 4);
+        s->tiles = e2d_tiles(N);
+        rc = dalloc(s->fields, e2d_state_floats(N) * 4);
         // 16 floats past the last material array: the staged kernel's
         // 16-byte chunks of the last row may extend into them
         if (rc == SM_OK) rc = dalloc(s->mat, (E2_NMAT * N + 16) * 4);
@@ -762,7 +788,7 @@ int sm_e2d_get_field_padded(sm_e2d *s, int comp, double *out)
     SM_CHECK(slot >= 0, SM_ERR_ARG, "sm_e2d_get_field_padded: component %d", comp);
     SM_CHECK(set_device(s->ctx) == SM_OK, SM_ERR_HIP, "hipSetDevice failed");
     size_t arr = (size_t)slot;
-    if (s->fused) arr += (s->step & 1) * E2_NSTATE;   // parity buffer holding step s->step
+    if (s->fused) arr += (size_t)s->cur * E2_NSTATE;
     const char *src = (const char *)s->fields.ptr + arr * s->N * s->elt;
     if (s->elt == 8) return read_back<double>(s, src, s->N, out);
     return read_back<float>(s, src, s->N, out);
@@ -939,6 +965,7 @@ int sm_e2d_batch_run(sm_e2d_batch *b, size_t nshots, sm_e2d *const *shots, const
     if (rc != SM_OK) return rc;
     if (b->group_bytes == 0) {
         rc = b->runner.run(d, b->ctx->stream, b->graph_steps);
+        for (size_t k = 0; k < nshots && rc == SM_OK; ++k) e2d_advance(shots[k], b->runner, nsteps[k]);
     } else {
         // longest runs first, packed greedily into groups whose footprint
         // stays within group_bytes (a larger shot runs alone); each group
@@ -949,11 +976,13 @@ int sm_e2d_batch_run(sm_e2d_batch *b, size_t nshots, sm_e2d *const *shots, const
         std::stable_sort(ord.begin(), ord.end(),
                          [&](size_t x, size_t y) { return nsteps[x] > nsteps[y]; });
         std::vector<E2dShot> g;
-        size_t acc = 0;
+        size_t acc = 0, done = 0;
         for (size_t q = 0; q <= nshots && rc == SM_OK; ++q) {
             const size_t fb = q < nshots ? shot_footprint(shots[ord[q]]) : 0;
             if (!g.empty() && (q == nshots || acc + fb > b->group_bytes)) {
                 rc = b->runner.run(g, b->ctx->stream, b->graph_steps);
+                for (; done < q && rc == SM_OK; ++done)
+                    e2d_advance(shots[ord[done]], b->runner, nsteps[ord[done]]);
                 g.clear();
                 acc = 0;
             }
@@ -965,7 +994,6 @@ int sm_e2d_batch_run(sm_e2d_batch *b, size_t nshots, sm_e2d *const *shots, const
     }
     if (rc != SM_OK) return rc;
     SM_HIP(hipStreamSynchronize(b->ctx->stream));
-    for (size_t k = 0; k < nshots; ++k) shots[k]->step += nsteps[k];
     return SM_OK;
 }
 
@@ -978,7 +1006,7 @@ int sm_e2d_batch_run_noalloc(sm_e2d_batch *b, size_t nshots, sm_e2d *const *shot
     rc = b->runner.run_static(d, b->ctx->device, b->ctx->stream);
     if (rc != SM_OK) return rc;
     SM_HIP(hipStreamSynchronize(b->ctx->stream));
-    for (size_t k = 0; k < nshots; ++k) shots[k]->step += nsteps[k];
+    for (size_t k = 0; k < nshots; ++k) e2d_advance(shots[k], b->runner, nsteps[k]);
     return SM_OK;
 }
 

@@ -14,6 +14,7 @@
 //              where it is not (pml.c:123); the total is x + z.
 // Neighbours off the padded grid read 0 (pml.c:58, 79).
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -152,8 +153,8 @@ e2d_fused_step(const E2dShot *__restrict__ shots, const int *__restrict__ bshot,
     // rows outside the grid are not loaded (0); cells outside [0, NZ) are
     // masked by the reader (jv), as the per-lane loads mask them.
     const int J0m = zt * E2D_OWN - 1;
-    const int par_off = (int)(S->st[it & 1] - S->st[0]);   // floats: 0 or E2_NSTATE*N
-    const auto Rall = rsrc(S->st[0], (2 * E2_NSTATE + E2_NSPLIT) * N4);
+    const int par_off = (int)(S->st[it & 1] - S->base);   // floats: 0 or E2_NSTATE*N
+    const auto Rall = rsrc(S->base, 2 * E2_NSTATE * N4);
     const auto Rmat16 = rsrc(S->mat, E2_NMAT * N4 + 64);
     u32x4 *const stage = s_stage + (STAGED ? w * 256 : 0);
     // float index (within its allocation) of field-row fr's first cell
@@ -453,6 +454,299 @@ e2d_fused_step(const E2dShot *__restrict__ shots, const int *__restrict__ bshot,
     else body(std::false_type{});
 }
 
+// ---------------------------------------------------------------------
+// Several steps per launch.
+// ---------------------------------------------------------------------
+// value of lane - 1 / lane + 1, 0 past the ends of the wave (DPP: a vector
+// instruction, no LDS)
+__device__ __forceinline__ float lane_m1(float x)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_p1(float x)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, true));
+}
+
+// Launch `launch` of K steps: a block of W waves holds a tile of E2D_TROWS W
+// rows by 64 z cells in registers (a wave E2D_TROWS rows, a lane one z cell)
+// and advances it up to K steps.  A step reaches one cell in each direction,
+// so K cells on every side of the tile are recomputed copies of the
+// neighbours' cells whose values go stale one ring a step; the rest is
+// owned and written.  z neighbours are the next lanes, x neighbours the
+// thread's other rows; rows on either side of a wave pass through LDS, two
+// barriers a step.  The expressions are those of e2d_fused_step, so both
+// give the same bits.  State and split fields are read from one buffer and
+// written to the other: the neighbours' halos read what this block advances.
+__global__ void __launch_bounds__(64 * E2D_TWAVES)
+e2d_tile_steps(const E2dShot *__restrict__ shots, const int *__restrict__ bshot, int nblocks, int launch, int K)
+{
+    constexpr int M = E2D_TROWS;
+    // LDS of a wave: what it passes to the next ones (txx of its last row,
+    // txz of its first, then vz of its last, vx of its first), its receivers,
+    // and the fields of the rows that have some
+    struct Wave {
+        float edge[4][64];
+        float rows[M][5][64];
+        int2 rcv[E2D_TRCV];
+    };
+    static_assert(sizeof(Wave) == E2D_TLDS, "LDS of a wave");
+    extern __shared__ __align__(16) unsigned char e2d_lds[];
+    Wave *const lds = (Wave *)e2d_lds;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int W = blockDim.x >> 6;
+    const int nb = gridDim.x;
+    const int logical = (int)(blockIdx.x & 7) * (nb >> 3) + (int)(blockIdx.x >> 3);
+    if (logical >= nblocks) return;
+    const E2dShot *S = shots + bshot[logical];
+    const int s0 = launch * K;
+    if (s0 >= S->nsteps) return;
+    const int nst = min(K, S->nsteps - s0);
+    const int q = logical - S->tblk0, tnz = S->tnz;
+    const int xt = q / tnz, zt = q - xt * tnz;
+    const int NX = S->NX, NZ = S->NZ, np = S->np, nx = S->nx, nz = S->nz;
+    const int J = zt * (64 - 2 * K) - K + lane;
+    const int I0 = xt * (M * W - 2 * K) - K + w * M;
+    const bool jv = J >= 0 && J < NZ;
+    const bool ownj = jv && lane >= K && lane < 64 - K;
+    const bool pzl = J < np || J >= np + nz;
+    auto rv = [&](int R) { return R >= 0 && R < NX; };
+    auto px = [&](int R) { return R < np || R >= np + nx; };
+    auto ownr = [&](int m) { return w * M + m >= K && w * M + m < M * W - K && rv(I0 + m); };
+    const unsigned N = S->N, N4 = N * 4u;
+    const auto Rin = rsrc(S->tst[launch & 1], E2_NSTATE * N4);
+    const auto Rout = rsrc(S->tst[(launch + 1) & 1], E2_NSTATE * N4);
+    const auto Rsi = rsrc(S->tss[launch & 1], E2_NSPLIT * N4);
+    const auto Rso = rsrc(S->tss[(launch + 1) & 1], E2_NSPLIT * N4);
+    const auto Rmat = rsrc(S->mat, E2_NMAT * N4);
+    const int it0 = S->it0 + s0;
+
+    // receivers at this wave's owned cells, compacted into LDS as (place in
+    // Wave::rows, trace column); more than the list holds are looked up per step
+    const int nrec = S->nrec, rmax = S->rmax;
+    const int4 *const rcv = S->rcv;
+    const int *const rrow = S->rrow;
+    float *const trace = S->trace;
+    const int row0 = it0 - S->rcv0;
+    int rcount = 0;
+    unsigned rmask = 0;
+    if (nrec) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            if (!ownr(m)) continue;
+            const int R = I0 + m, e1 = cld(rrow + R + 1);
+            for (int e0 = cld(rrow + R); e0 < e1; e0 += 64) {
+                const int e = e0 + lane;
+                const int4 r = e < e1 ? rcv[e] : make_int4(-1, 0, 0, 0);
+                const int l = r.x - R * NZ - J + lane;   // lane of the receiver's cell
+                const bool mine = e < e1 && l >= K && l < 64 - K;
+                const unsigned long long bal = __ballot(mine);
+                if (bal) rmask |= 1u << m;
+                const int at = rcount + __popcll(bal & ((1ull << lane) - 1));
+                if (mine && at < E2D_TRCV) lds[w].rcv[at] = make_int2((m * 5 + r.y) * 64 + l, r.z);
+                rcount += __popcll(bal);
+            }
+        }
+    }
+    const bool rlist = rcount <= E2D_TRCV;
+    const int2 rcv1 = lane < rcount && lane < E2D_TRCV ? lds[w].rcv[lane] : make_int2(0, 0);
+    // sources in this wave's rows (halo copies included)
+    const int nsrc = S->nsrc;
+    const int4 *const src = S->src;
+    const float *const sfct = S->sfct;
+    const int sp0 = nsrc ? cld(S->srow + min(max(I0, 0), NX)) : 0;
+    const int sp1 = nsrc ? cld(S->srow + min(max(I0 + M, 0), NX)) : 0;
+    const int4 src1 = sp1 > sp0 ? cld(src + sp0) : make_int4(0, 0, 0, 0);
+    const int src_row = src1.x / NZ - I0;
+    const bool src_lane = sp1 > sp0 && J == src1.x % NZ;
+
+    const bool pmlw = __any(jv && pzl) || (I0 < np && I0 + M > 0) || (I0 + M > np + nx && I0 < NX);
+    auto body = [&](auto pml_tag) {
+        constexpr bool PML = decltype(pml_tag)::value;
+        float vx[M], vz[M], sxx[M], szz[M], sxz[M], cb[M], cbm[M], la[M], l2m[M], mu[M];
+        float a[PML ? M : 1][E2_NSTATE - E2_VXX + E2_NSPLIT];
+        bool pm[M];
+        float2 xi[PML ? M : 1], xh[PML ? M : 1], zi, zh;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int R = I0 + m;
+            const unsigned o = rv(R) && jv ? ((unsigned)R * NZ + J) * 4u : OFF_NONE;
+            sxx[m] = bld(Rin, o, E2_TXX * N4);
+            szz[m] = bld(Rin, o, E2_TZZ * N4);
+            sxz[m] = bld(Rin, o, E2_TXZ * N4);
+            vx[m] = bld(Rin, o, E2_VX * N4);
+            vz[m] = bld(Rin, o, E2_VZ * N4);
+            cb[m] = bld(Rmat, o, E2_CB * N4);
+            cbm[m] = bld(Rmat, o, E2_CBM * N4);
+            la[m] = bld(Rmat, o, E2_CLA * N4);
+            l2m[m] = bld(Rmat, o, E2_CL2M * N4);
+            mu[m] = bld(Rmat, o, E2_CMU * N4);
+            if constexpr (PML) {
+                pm[m] = rv(R) && (px(R) || pzl);
+                const unsigned op = pm[m] ? o : OFF_NONE;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) a[m][c] = bld(Rin, op, (E2_VXX + c) * N4);
+#pragma unroll
+                for (int c = 0; c < E2_NSPLIT; ++c) a[m][4 + c] = bld(Rsi, op, c * N4);
+                const float2 *t = (const float2 *)S->dmp;
+                const int Rc = min(max(R, 0), NX - 1);
+                xi[m] = cld(t + Rc);
+                xh[m] = cld(t + NX + Rc);
+            }
+        }
+        if constexpr (PML) {
+            const float2 *t = (const float2 *)S->dmp + 2 * NX;
+            const int Jc = min(max(J, 0), NZ - 1);
+            zi = t[Jc];
+            zh = t[NZ + Jc];
+        }
+        for (int k = 0; k < nst; ++k) {
+            const int it = it0 + k;
+            // the one source of a wave: its sample is on its way early
+            const float inc1 = sp1 == sp0 + 1 && it < src1.z ? cld(sfct + src1.w + it) : 0.f;
+            lds[w].edge[0][lane] = sxx[M - 1];
+            lds[w].edge[1][lane] = sxz[0];
+            __syncthreads();
+            const float sxx_u = w > 0 ? lds[w - 1].edge[0][lane] : 0.f;
+            const float sxz_d = w + 1 < W ? lds[w + 1].edge[1][lane] : 0.f;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                {
+                    const float dxs = sxx[m] - (m ? sxx[m - 1] : sxx_u);
+                    const float dzs = sxz[m] - lane_m1(sxz[m]);
+                    vx[m] = vx[m] + cb[m] * (dxs + dzs);
+                    if constexpr (PML) {
+                        a[m][0] = xi[m].x * a[m][0] + xi[m].y * (cb[m] * dxs);
+                        a[m][1] = zi.x * a[m][1] + zi.y * (cb[m] * dzs);
+                        if (pm[m]) vx[m] = a[m][0] + a[m][1];
+                    }
+                }
+                {
+                    const float dxs = (m + 1 < M ? sxz[m + 1 < M ? m + 1 : m] : sxz_d) - sxz[m];
+                    const float dzs = lane_p1(szz[m]) - szz[m];
+                    vz[m] = vz[m] + cbm[m] * (dxs + dzs);
+                    if constexpr (PML) {
+                        a[m][2] = xh[m].x * a[m][2] + xh[m].y * (cbm[m] * dxs);
+                        a[m][3] = zh.x * a[m][3] + zh.y * (cbm[m] * dzs);
+                        if (pm[m]) vz[m] = a[m][2] + a[m][3];
+                    }
+                }
+            }
+            lds[w].edge[2][lane] = vz[M - 1];
+            lds[w].edge[3][lane] = vx[0];
+            __syncthreads();
+            const float vz_u = w > 0 ? lds[w - 1].edge[2][lane] : 0.f;
+            const float vx_d = w + 1 < W ? lds[w + 1].edge[3][lane] : 0.f;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const float dvxx = (m + 1 < M ? vx[m + 1 < M ? m + 1 : m] : vx_d) - vx[m];
+                const float dvzz = vz[m] - lane_m1(vz[m]);
+                const float dvxz = lane_p1(vx[m]) - vx[m];
+                const float dvzx = vz[m] - (m ? vz[m - 1] : vz_u);
+                sxx[m] = sxx[m] + (l2m[m] * dvxx + la[m] * dvzz);
+                szz[m] = szz[m] + (l2m[m] * dvzz + la[m] * dvxx);
+                sxz[m] = sxz[m] + mu[m] * (dvxz + dvzx);
+                if constexpr (PML) {
+                    float *t = a[m] + 4;
+                    t[E2_TXXX] = xh[m].x * t[E2_TXXX] + xh[m].y * (l2m[m] * dvxx);
+                    t[E2_TXXZ] = zi.x * t[E2_TXXZ] + zi.y * (la[m] * dvzz);
+                    t[E2_TZZX] = xh[m].x * t[E2_TZZX] + xh[m].y * (la[m] * dvxx);
+                    t[E2_TZZZ] = zi.x * t[E2_TZZZ] + zi.y * (l2m[m] * dvzz);
+                    t[E2_TXZX] = xi[m].x * t[E2_TXZX] + xi[m].y * (mu[m] * dvzx);
+                    t[E2_TXZZ] = zh.x * t[E2_TXZZ] + zh.y * (mu[m] * dvxz);
+                    if (pm[m]) {
+                        sxx[m] = t[E2_TXXX] + t[E2_TXXZ];
+                        szz[m] = t[E2_TZZX] + t[E2_TZZZ];
+                        sxz[m] = t[E2_TXZX] + t[E2_TXZZ];
+                    }
+                }
+            }
+            // add_src (src.c:170-184) after both phases
+            auto add = [&](int4 e, int m, float inc) {
+                if (e.y == SM_SX || e.y == SM_BULK) sxx[m] += inc;
+                if (e.y == SM_SZ || e.y == SM_BULK) szz[m] += inc;
+                if (e.y == SM_SXZ) sxz[m] += inc;
+            };
+            if (sp1 == sp0 + 1) {
+                if (it < src1.z) {
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+                        if (m == src_row && src_lane) add(src1, m, inc1);
+                }
+            } else {
+                for (int e = sp0; e < sp1; ++e) {
+                    const int4 r = cld(src + e);
+                    if (it >= r.z) continue;
+                    const float inc = cld(sfct + r.w + it);
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+                        if (rv(I0 + m) && jv && r.x == (I0 + m) * NZ + J) add(r, m, inc);
+                }
+            }
+            // receivers (e_iso.c:641-669 samples after add_src): the rows with
+            // some go through LDS, a lane takes a receiver (the wave's own
+            // LDS, so no barrier; a branch per lane and field cost 4500
+            // cycles a step)
+            const int row = row0 + k;
+            if (rmask && row >= 0 && row < rmax) {
+                float *tr = trace + (size_t)row * nrec;
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    if (!(rmask >> m & 1)) continue;
+                    float (*f)[64] = lds[w].rows[m];
+                    f[0][lane] = vx[m];
+                    f[1][lane] = vz[m];
+                    f[2][lane] = sxx[m];
+                    f[3][lane] = szz[m];
+                    f[4][lane] = sxz[m];
+                }
+                __builtin_amdgcn_wave_barrier();
+                const float *f = &lds[w].rows[0][0][0];
+                if (rlist) {
+                    if (lane < rcount) tr[rcv1.y] = f[rcv1.x];
+                    for (int e = lane + 64; e < rcount; e += 64) {
+                        const int2 r = lds[w].rcv[e];
+                        tr[r.y] = f[r.x];
+                    }
+                } else {
+                    for (int m = 0; m < M; ++m) {
+                        if (!(rmask >> m & 1)) continue;
+                        const int R = I0 + m, e1 = cld(rrow + R + 1);
+                        for (int e = cld(rrow + R) + lane; e < e1; e += 64) {
+                            const int4 r = rcv[e];
+                            const int l = r.x - R * NZ - J + lane;
+                            if (l >= K && l < 64 - K) tr[r.z] = f[(m * 5 + r.y) * 64 + l];
+                        }
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int R = I0 + m;
+            const unsigned o = ownr(m) && ownj ? ((unsigned)R * NZ + J) * 4u : OFF_NONE;
+            bst(Rout, o, E2_VX * N4, vx[m]);
+            bst(Rout, o, E2_VZ * N4, vz[m]);
+            bst(Rout, o, E2_TXX * N4, sxx[m]);
+            bst(Rout, o, E2_TZZ * N4, szz[m]);
+            bst(Rout, o, E2_TXZ * N4, sxz[m]);
+            if constexpr (PML) {
+                const unsigned op = pm[m] ? o : OFF_NONE;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) bst(Rout, op, (E2_VXX + c) * N4, a[m][c]);
+#pragma unroll
+                for (int c = 0; c < E2_NSPLIT; ++c) bst(Rso, op, c * N4, a[m][4 + c]);
+            }
+        }
+    };
+    // (a wave-uniform branch: every wave of a block passes the same number
+    // of barriers in either form)
+    if (pmlw) body(std::true_type{});
+    else body(std::false_type{});
+}
+
 __global__ void e2d_base_set(int *base, int value, int add)
 {
     if (threadIdx.x == 0) *base = add ? *base + value : value;
@@ -612,8 +906,118 @@ int E2dRunner::launch_all(const std::vector<E2dShot> &shots, const std::vector<i
     return SM_OK;
 }
 
+namespace {
+
+int tile_blocks(const E2dShot &d, E2dTile t, int *tnz)
+{
+    const int ownx = E2D_TROWS * t.waves - 2 * t.steps, ownz = 64 - 2 * t.steps;
+    *tnz = (d.NZ + ownz - 1) / ownz;
+    return *tnz * ((d.NX + ownx - 1) / ownx);
+}
+
+// Waves and steps of the tile kernel for a list of shots; steps 0: one launch
+// a step instead, for a single step (7.3 against 7.6 us on 440^2 cells) and
+// for grids without a second split buffer.  Estimate of a launch in us, from
+// the kernel's clocks: 6 for the launch, the first loads and the last stores;
+// a step 0.5 for its two barriers and LDS trips plus 0.135 for every wave of
+// the fullest compute unit (320 vector instructions in the layers); tiles with
+// their halos at 6 TB/s.  Measured: 440^2, 1000 steps, 8 waves: 4 steps 3.56
+// ms, 6 3.05, 7 2.86 (225 blocks), 8 3.00 (280 blocks, two on some units); 24
+// shots of 10 M cells in all: 8 waves 7 steps 13.7 ms, 16 waves 8 steps 13.0.
+E2dTile tile_shape(const std::vector<E2dShot> &shots, int cus)
+{
+    E2dTile best;
+    int most = 0;
+    for (const E2dShot &d : shots) {
+        if (!d.tss[1]) return best;
+        most = std::max(most, d.nsteps);
+    }
+    if (most < 2) return best;
+    double least = 1e30;
+    for (int W : {4, 6, 8, 12, 16})
+        for (int K = 2; K <= 14 && 2 * K < E2D_TROWS * W; ++K) {
+            const E2dTile t{W, K};
+            double blocks = 0;
+            int tnz;
+            for (const E2dShot &d : shots) blocks += tile_blocks(d, t, &tnz);
+            const double launch = 6.0 + K * (0.5 + 0.135 * W * std::ceil(blocks / cus)) +
+                                  blocks * (64.0 * E2D_TROWS * W * 40.0) / 6e6;
+            const double total = launch * ((most + K - 1) / K);
+            if (total < least) { least = total; best = t; }
+        }
+    return best;
+}
+
+}  // namespace
+
+int E2dRunner::run_tiles(std::vector<E2dShot> &shots, hipStream_t st)
+{
+    std::stable_sort(shots.begin(), shots.end(),
+                     [](const E2dShot &a, const E2dShot &b) { return a.nsteps > b.nsteps; });
+    const size_t n = shots.size();
+    std::vector<int> pref(n + 1, 0);
+    for (size_t i = 0; i < n; ++i) {
+        shots[i].tblk0 = pref[i];
+        const long long next = (long long)pref[i] + tile_blocks(shots[i], tile_, &shots[i].tnz);
+        SM_CHECK(next < (1ll << 30), SM_ERR_ARG, "batch too large: %lld blocks", next);
+        pref[i + 1] = (int)next;
+    }
+    const size_t tab_bytes = (n * sizeof(E2dShot) + 255) & ~(size_t)255;
+    std::vector<unsigned char> host(tab_bytes + (size_t)pref[n] * sizeof(int), 0);
+    std::memcpy(host.data(), shots.data(), n * sizeof(E2dShot));
+    int *bs = (int *)(host.data() + tab_bytes);
+    for (size_t i = 0; i < n; ++i)
+        for (int q = pref[i]; q < pref[i + 1]; ++q) bs[q] = (int)i;
+    // (captured graphs read the table's memory)
+    drop_graphs();
+    last_tab_bytes_ = 0;
+    int rc = ensure(host.size());
+    if (rc != SM_OK) return rc;
+    SM_HIP(hipMemcpyAsync(table_, host.data(), host.size(), hipMemcpyHostToDevice, st));
+    SM_HIP(hipStreamSynchronize(st));
+    hipEvent_t t0 = nullptr, t1 = nullptr;
+    if (timing) {
+        SM_HIP(hipEventCreate(&t0));
+        SM_HIP(hipEventCreate(&t1));
+        SM_HIP(hipEventRecord(t0, st));
+    }
+    const int total = shots[0].nsteps;
+    size_t m = n;
+    for (int l = 0; l * tile_.steps < total; ++l) {
+        while (shots[m - 1].nsteps <= l * tile_.steps) --m;
+        const int nblk = pref[m];
+        e2d_tile_steps<<<(nblk + 7) & ~7, 64 * tile_.waves, (size_t)tile_.waves * E2D_TLDS, st>>>(
+            (const E2dShot *)table_, (const int *)((const char *)table_ + tab_bytes), nblk, l, tile_.steps);
+    }
+    SM_HIP(hipGetLastError());
+    if (timing) {
+        SM_HIP(hipEventRecord(t1, st));
+        SM_HIP(hipEventSynchronize(t1));
+        float ms = 0.f;
+        SM_HIP(hipEventElapsedTime(&ms, t0, t1));
+        (void)hipEventDestroy(t0);
+        (void)hipEventDestroy(t1);
+        ms_total += ms;
+        launches += (size_t)total;
+    }
+    return SM_OK;
+}
+
 int E2dRunner::run(std::vector<E2dShot> shots, hipStream_t st, int graph_steps)
 {
+    shots.erase(std::remove_if(shots.begin(), shots.end(), [](const E2dShot &d) { return d.nsteps <= 0; }),
+                shots.end());
+    tile_ = E2dTile{};
+    if (shots.empty()) return SM_OK;
+    if (!cus_) {
+        int dev = 0;
+        SM_HIP(hipGetDevice(&dev));
+        SM_HIP(hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev));
+        SM_HIP(hipFuncSetAttribute((const void *)e2d_tile_steps, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   E2D_TWAVES * E2D_TLDS));
+    }
+    tile_ = tile_shape(shots, cus_);
+    if (tile_.steps) return run_tiles(shots, st);
     std::vector<int> pref;
     std::vector<unsigned char> host;
     size_t tab_bytes = 0;
@@ -697,6 +1101,7 @@ int E2dRunner::run_static(std::vector<E2dShot> shots, int device, hipStream_t st
     }
     SM_CHECK(scratch, SM_ERR_STATE, "allocation-free batch: no scratch address for device %d "
              "(the context was not created by sm_ctx_create)", device);
+    tile_ = E2dTile{};
     std::vector<int> pref;
     std::vector<unsigned char> host;
     size_t tab_bytes = 0;
