@@ -318,9 +318,9 @@ int sm_e2d_get_timing(const sm_e2d *s, double *ms_total, size_t *launches);
 
 /* ------------------------------------------------------------------ */
 /* Batches of independent 2D shots (no counterpart in the reference,   */
-/* which runs one shot per process).  One launch advances every shot      */
-/* that still has steps to run, by several steps at a time.  Each shot's results are those of running   */
-/* it alone with sm_e2d_run.                                            */
+/* which runs one shot per process).  One launch advances every shot    */
+/* that still has steps to run, by several steps at a time.  Each       */
+/* shot's results are those of running it alone with sm_e2d_run.        */
 /* ------------------------------------------------------------------ */
 typedef struct sm_e2d_batch sm_e2d_batch;
 int sm_e2d_batch_create(sm_ctx *ctx, sm_e2d_batch **out);

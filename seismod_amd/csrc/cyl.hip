@@ -57,7 +57,29 @@ struct CylDev {
     const int *stype;
     const T *sfct;
     int64_t it;
+    // tiles of 64 z by 4 r cells along z, their number; receivers in tile
+    // order: padded cell, component, trace column, first of each tile;
+    // row of the trace to record this step (< 0: none)
+    int gx, nblk;
+    int nrec;
+    const int64_t *ridx;
+    const int *rcomp, *rcol, *rstart;
+    T *trace;
+    int64_t row;
 };
+
+// tile of this block: every XCD takes a range of consecutive tiles, so that
+// tiles next to each other along z share an L2.  Rows need not start on cache
+// lines, and with neighbours on other XCDs the lines at both ends of a
+// wave's 64 cells were read and written by two of them (with the receivers in
+// the stress kernel 153 -> 144 us a step on 1020 x 4040 FP32 cells; rows of
+// 16160 bytes).
+template <typename T>
+__device__ __forceinline__ int cyl_tile(const CylDev<T> &d)
+{
+    const int per = (int)(gridDim.x >> 3);
+    return (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+}
 
 template <typename T>
 struct Coef {
@@ -143,12 +165,13 @@ __device__ __forceinline__ T *zmem(const CylDev<T> &d, int q, int i, int j, int 
 #define FLD(q, i, j) d.f[q][(size_t)(i) * d.nz2 + (j)]
 #define MAT(q, c) d.m[(size_t)(q) * N + (c)]
 
-template <typename T>
-__global__ void __launch_bounds__(256) cyl_velocity(CylDev<T> d)
+// TOR: the torsional fields (v_theta, tau_rtheta, tau_thetaz) take part.  In
+// mode 0 they do not couple to the others, so without a source that ever
+// excited them they are 0 and stay 0 (a step on 1020 x 4040 FP32 cells 144 ->
+// 77 us, FP64 249 -> 152: 17 of 26 values a cell, and half as many in flight).
+template <typename T, bool TOR>
+__device__ __forceinline__ void velocity_cell(const CylDev<T> &d, int i, int j)
 {
-    const int j = blockIdx.x * 64 + threadIdx.x;
-    const int i = blockIdx.y * 4 + threadIdx.y;
-    if (i >= d.nx2 || j >= d.nz2) return;
     const size_t N = (size_t)d.nx2 * d.nz2;
     const size_t c = (size_t)i * d.nz2 + j;
     const T dx = d.dx, dz = d.dz, dt = d.dt;
@@ -192,7 +215,7 @@ __global__ void __launch_bounds__(256) cyl_velocity(CylDev<T> d)
     if (i + 1 < d.nx2) {
         const T ihdx = ((T)i + T(0.5)) * dx;
         // ---- v_theta (propagate.c:2815-2906, 3479-3585)
-        if (j + 1 < d.nz2) {
+        if (TOR && j + 1 < d.nz2) {
             const Coef<T> kr = rc_half(d, i, d.nx - 1);
             const Coef<T> kz = zc_half(d, j, jb_half);
             T ddz = (FLD(C_TTZ, i, j + 1) - FLD(C_TTZ, i, j)) / dz;
@@ -248,12 +271,9 @@ __global__ void __launch_bounds__(256) cyl_velocity(CylDev<T> d)
     }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) cyl_stress(CylDev<T> d)
+template <typename T, bool TOR>
+__device__ __forceinline__ void stress_cell(const CylDev<T> &d, int i, int j)
 {
-    const int j = blockIdx.x * 64 + threadIdx.x;
-    const int i = blockIdx.y * 4 + threadIdx.y;
-    if (i >= d.nx2 || j >= d.nz2) return;
     const size_t N = (size_t)d.nx2 * d.nz2;
     const size_t c = (size_t)i * d.nz2 + j;
     const T dx = d.dx, dz = d.dz, dt = d.dt;
@@ -290,7 +310,7 @@ __global__ void __launch_bounds__(256) cyl_stress(CylDev<T> d)
             }
         }
         // ---- tau_thetaz (propagate.c:3249-3310, 4010-4088)
-        if (j >= 1) {
+        if (TOR && j >= 1) {
             const Coef<T> kz = zc_node(d, j);
             const T dvt = FLD(C_VT, i, j) - FLD(C_VT, i, j - 1);
             if (n == 0) {
@@ -324,7 +344,7 @@ __global__ void __launch_bounds__(256) cyl_stress(CylDev<T> d)
         FLD(C_TRZ, i, j) += dt * MAT(M_MU, c) * (ddz + ddr);
     }
     // ---- tau_rtheta (propagate.c:3215-3247, 3958-4008)
-    if (i >= 1 || (n % 2)) {
+    if (TOR && (i >= 1 || (n % 2))) {
         if (i == 0) {
             FLD(C_TRT, i, j) += dt * MAT(M_MUJ, c) * ((FLD(C_VT, i, j) - -FLD(C_VT, i, j)) / dx);
         } else {
@@ -360,16 +380,13 @@ __global__ void __launch_bounds__(256) cyl_stress(CylDev<T> d)
 // receiver values after step it (divergence and curl evaluated at the
 // receiver's cell with propagate.c:4090-4119's expressions; cells outside
 // their ranges read 0 as the reference's zero-initialised arrays do)
+// the recorded value of component comp at padded cell c
 template <typename T>
-__global__ void cyl_gather(CylDev<T> d, int nrec, const int64_t *ridx, const int *rcomp, T *trace,
-                           int64_t row)
+__device__ __forceinline__ T recorded(const CylDev<T> &d, int64_t c, int comp)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrec) return;
-    const int64_t c = ridx[r];
     const int i = (int)(c / d.nz2), j = (int)(c % d.nz2);
     T v = T(0);
-    switch (rcomp[r]) {
+    switch (comp) {
     case SM_VR: v = d.f[C_VR][c]; break;
     case SM_VT: v = d.f[C_VT][c]; break;
     case SM_VZ: v = d.f[C_VZ][c]; break;
@@ -393,7 +410,36 @@ __global__ void cyl_gather(CylDev<T> d, int nrec, const int64_t *ridx, const int
         break;
     default: break;
     }
-    trace[(size_t)row * nrec + r] = v;
+    return v;
+}
+
+template <typename T, bool TOR>
+__global__ void __launch_bounds__(256) cyl_velocity(const CylDev<T> d)
+{
+    const int t = cyl_tile(d);
+    if (t >= d.nblk) return;
+    const int y = t / d.gx, i = y * 4 + (int)threadIdx.y, j = (t - y * d.gx) * 64 + (int)threadIdx.x;
+    if (i < d.nx2 && j < d.nz2) velocity_cell<T, TOR>(d, i, j);
+}
+
+// The stresses, then the receivers in the block's own tile: the velocities
+// are final and the tile's stresses its own block's, so only a block barrier
+// orders them, and the separate gather launch a step (4.7 us) is not needed.
+template <typename T, bool TOR>
+__global__ void __launch_bounds__(256) cyl_stress(const CylDev<T> d)
+{
+    const int t = cyl_tile(d);
+    if (t >= d.nblk) return;
+    const int y = t / d.gx, i = y * 4 + (int)threadIdx.y, j = (t - y * d.gx) * 64 + (int)threadIdx.x;
+    if (i < d.nx2 && j < d.nz2) stress_cell<T, TOR>(d, i, j);
+    if (d.row < 0) return;
+    const int r1 = d.rstart[t + 1];
+    int r = d.rstart[t];
+    if (r == r1) return;
+    __threadfence_block();
+    __syncthreads();
+    for (r += (int)(threadIdx.y * 64 + threadIdx.x); r < r1; r += 256)
+        d.trace[(size_t)d.row * d.nrec + d.rcol[r]] = recorded(d, d.ridx[r], d.rcomp[r]);
 }
 
 #undef FLD
@@ -410,6 +456,8 @@ struct sm_cyl {
     size_t nx2 = 0, nz2 = 0, N = 0, elt = 8;
     sm_dbuf fields, mem, mat, tab, src, rcv, trace;
     size_t nsrc = 0, nrec = 0, max_steps = 0, rcv_step0 = 0, step = 0;
+    bool src_tor = false;           // a source excites the torsional fields
+    bool torsional = false;         // they may be nonzero
     bool timing = false;            // HIP events around each step's two launches
     double timed_ms = 0.0;
     size_t timed_steps = 0;
@@ -426,6 +474,9 @@ size_t mem_count(size_t np, size_t nx2, size_t nz2)
 {
     return np ? (size_t)R_NM * (np + 1) * nz2 + (size_t)Z_NM * nx2 * (2 * np + 1) : 0;
 }
+
+// tiles of 64 z by 4 r cells
+size_t tiles(size_t nx2, size_t nz2) { return (nz2 + 63) / 64 * ((nx2 + 3) / 4); }
 
 template <typename T>
 CylDev<T> view(sm_cyl *s, int64_t it)
@@ -445,6 +496,16 @@ CylDev<T> view(sm_cyl *s, int64_t it)
     d.stype = d.src ? (const int *)(d.src + 3 * s->nsrc) : nullptr;
     d.sfct = d.src ? (const T *)(d.src + 4 * s->nsrc) : nullptr;
     d.it = it;
+    d.gx = (int)((s->nz2 + 63) / 64);
+    d.nblk = (int)tiles(s->nx2, s->nz2);
+    d.nrec = (int)s->nrec;
+    d.ridx = (const int64_t *)s->rcv.ptr;
+    d.rcomp = d.ridx ? (const int *)(d.ridx + s->nrec) : nullptr;
+    d.rcol = d.rcomp ? d.rcomp + s->nrec : nullptr;
+    d.rstart = d.rcol ? d.rcol + s->nrec : nullptr;
+    d.trace = (T *)s->trace.ptr;
+    const size_t q = (size_t)it;
+    d.row = s->nrec && q >= s->rcv_step0 && q - s->rcv_step0 < s->max_steps ? (int64_t)(q - s->rcv_step0) : -1;
     return d;
 }
 
@@ -473,9 +534,8 @@ int run(sm_cyl *s, size_t nsteps)
 {
     hipStream_t st = s->ctx->stream;
     const dim3 blk(64, 4, 1);
-    const dim3 grd((unsigned)((s->nz2 + 63) / 64), (unsigned)((s->nx2 + 3) / 4), 1);
-    const int64_t *ridx = (const int64_t *)s->rcv.ptr;
-    const int *rcomp = ridx ? (const int *)(ridx + s->nrec) : nullptr;
+    const unsigned grd = (unsigned)((tiles(s->nx2, s->nz2) + 7) / 8 * 8);
+    s->torsional = s->torsional || s->p.mode != 0 || s->src_tor;
     StepEvents te;
     if (s->timing) {
         te.ev.assign(2 * nsteps, nullptr);
@@ -485,12 +545,14 @@ int run(sm_cyl *s, size_t nsteps)
         const size_t it = s->step + k;
         CylDev<T> d = view<T>(s, (int64_t)it);
         if (s->timing) SM_HIP(hipEventRecord(te.ev[2 * k], st));
-        cyl_velocity<T><<<grd, blk, 0, st>>>(d);
-        cyl_stress<T><<<grd, blk, 0, st>>>(d);
+        if (s->torsional) {
+            cyl_velocity<T, true><<<grd, blk, 0, st>>>(d);
+            cyl_stress<T, true><<<grd, blk, 0, st>>>(d);
+        } else {
+            cyl_velocity<T, false><<<grd, blk, 0, st>>>(d);
+            cyl_stress<T, false><<<grd, blk, 0, st>>>(d);
+        }
         if (s->timing) SM_HIP(hipEventRecord(te.ev[2 * k + 1], st));
-        if (s->nrec && it >= s->rcv_step0 && it - s->rcv_step0 < s->max_steps)
-            cyl_gather<T><<<(unsigned)((s->nrec + 255) / 256), 256, 0, st>>>(
-                d, (int)s->nrec, ridx, rcomp, (T *)s->trace.ptr, (int64_t)(it - s->rcv_step0));
     }
     SM_HIP(hipGetLastError());
     s->step += nsteps;
@@ -544,7 +606,7 @@ size_t sm_cyl_bytes_needed(const sm_cyl_params *p, size_t nrec, size_t max_steps
     const size_t e = p->storage == SM_STORE_F64 ? 8 : 4;
     const size_t nx2 = p->nx + p->np, nz2 = p->nz + 2 * p->np, N = nx2 * nz2;
     return e * ((C_NF + M_NMAT) * N + mem_count(p->np, nx2, nz2) + 15 * (p->np + 1) +
-                nrec * max_steps) + 12 * nrec;
+                nrec * max_steps) + (nrec ? 16 * nrec + 4 * (tiles(nx2, nz2) + 1) : 0);
 }
 
 int sm_cyl_create(sm_ctx *ctx, const sm_cyl_params *pp, const double *vp, const double *vs,
@@ -715,6 +777,8 @@ int sm_cyl_set_sources(sm_cyl *s, size_t nsrc, const int *type, const size_t *id
     SM_HIP(hipStreamSynchronize(s->ctx->stream));
     dfree(s->src);
     s->nsrc = 0;
+    s->src_tor = false;
+    for (size_t k = 0; k < nsrc; ++k) s->src_tor = s->src_tor || type[k] == SM_FT;
     if (nsrc == 0) return SM_OK;
     const size_t bytes = 4 * nsrc * sizeof(int64_t) + total * s->elt;
     int rc = dalloc(s->src, bytes);
@@ -759,13 +823,29 @@ int sm_cyl_set_receivers(sm_cyl *s, size_t nrec, const size_t *idx, const int *c
     s->nrec = 0;
     s->max_steps = 0;
     if (nrec == 0 || max_steps == 0) return SM_OK;
-    int rc = dalloc(s->rcv, nrec * (sizeof(int64_t) + sizeof(int)));
+    // in tile order: cells, components, trace columns, first of each tile
+    const size_t nt = tiles(s->nx2, s->nz2), gx = (s->nz2 + 63) / 64;
+    auto tile = [&](size_t r) { return idx[r] / s->nz2 / 4 * gx + idx[r] % s->nz2 / 64; };
+    std::vector<size_t> order(nrec);
+    for (size_t r = 0; r < nrec; ++r) order[r] = r;
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return tile(a) < tile(b); });
+    const size_t bytes = nrec * (sizeof(int64_t) + 2 * sizeof(int)) + (nt + 1) * sizeof(int);
+    int rc = dalloc(s->rcv, bytes);
     if (rc == SM_OK) rc = dalloc(s->trace, nrec * max_steps * s->elt);
     if (rc != SM_OK) { dfree(s->rcv); dfree(s->trace); return rc; }
-    std::vector<unsigned char> hb(nrec * (sizeof(int64_t) + sizeof(int)));
+    std::vector<unsigned char> hb(bytes);
     int64_t *hi = (int64_t *)hb.data();
-    int *hc = (int *)(hi + nrec);
-    for (size_t r = 0; r < nrec; ++r) { hi[r] = (int64_t)idx[r]; hc[r] = comp[r]; }
+    int *hc = (int *)(hi + nrec), *hcol = hc + nrec, *hs = hcol + nrec;
+    for (size_t q = 0; q < nrec; ++q) {
+        const size_t r = order[q];
+        hi[q] = (int64_t)idx[r];
+        hc[q] = comp[r];
+        hcol[q] = (int)r;
+    }
+    for (size_t t = 0, q = 0; t <= nt; ++t) {
+        while (q < nrec && tile(order[q]) < t) ++q;
+        hs[t] = (int)q;
+    }
     SM_HIP(hipMemcpyAsync(s->rcv.ptr, hb.data(), hb.size(), hipMemcpyHostToDevice, s->ctx->stream));
     SM_HIP(hipMemsetAsync(s->trace.ptr, 0, s->trace.bytes, s->ctx->stream));
     SM_HIP(hipStreamSynchronize(s->ctx->stream));
@@ -840,6 +920,7 @@ int sm_cyl_reset(sm_cyl *s)
     SM_HIP(hipStreamSynchronize(st));
     s->step = 0;
     s->rcv_step0 = 0;
+    s->torsional = false;
     return SM_OK;
 }
 
