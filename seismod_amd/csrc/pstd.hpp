@@ -120,6 +120,38 @@ __device__ __forceinline__ T layer_fix(const Layer<T> &L, T d, int i, int j, int
     return out;
 }
 
+// Runge-Kutta inputs of one cell: the step-start values s and the
+// accumulated values w of NF state components.  A stage kernel loads every
+// input of its cell before it stores anything: the state, derivative and
+// memory-variable buffers may alias as far as the compiler knows, so a load
+// after a store waits its turn, and a cell's inputs then arrive one memory
+// round trip after the other.  (Bound by memory: an SH stage of 1040^2 FP32
+// moves its 138 MB at 5.6 TB/s.  Measured per launch, loads in place, all
+// loads first, and with the cells of cell_of_thread: sh_stage 1040^2 FP32
+// 27.9, 26.7, 24.6 us; ve_stage 469 x 363 FP64 22.7, 21.2, 18.8; pve_stage
+// 1040^2 FP32 52.4, 51.9, 49.4, 640 x 480 FP64 VTI 36.0, 37.0, 33.1.)
+template <typename T, int NF>
+struct RkCell {
+    T s[NF], w[NF];
+    __device__ __forceinline__ void load(const T *ws, const T *wa, int acc, size_t N, size_t n)
+    {
+#pragma unroll
+        for (int c = 0; c < NF; ++c) s[c] = ws[c * N + n];
+#pragma unroll
+        for (int c = 0; c < NF; ++c) w[c] = acc ? wa[c * N + n] : s[c];
+    }
+    // wt = s + a d (if set_t), w = w + b d
+    __device__ __forceinline__ void store(T *wo, T *wt, int set_t, T a, T b, const T *d, size_t N, size_t n) const
+    {
+        if (set_t) {
+#pragma unroll
+            for (int c = 0; c < NF; ++c) wt[c * N + n] = s[c] + a * d[c];
+        }
+#pragma unroll
+        for (int c = 0; c < NF; ++c) wo[c * N + n] = w[c] + b * d[c];
+    }
+};
+
 // complex multiply by the multiplier of bin l % m (ROWS false) or l / m
 template <typename T, bool ROWS>
 __global__ void pstd_kmul(Cx<T> *o, const Cx<T> *k, unsigned m, size_t n)
@@ -131,6 +163,15 @@ __global__ void pstd_kmul(Cx<T> *o, const Cx<T> *k, unsigned m, size_t n)
 }
 
 inline unsigned blocks(size_t n, unsigned bs = 256) { return (unsigned)((n + bs - 1) / bs); }
+
+// blocks of a pointwise kernel over n cells, a multiple of the 8 XCDs, and
+// the cell of a thread: every XCD takes one range of consecutive cells, the
+// rows whose z derivatives it transforms
+inline unsigned cell_blocks(size_t n) { return (blocks(n) + 7) / 8 * 8; }
+__device__ __forceinline__ unsigned cell_of_thread()
+{
+    return ((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) * blockDim.x + threadIdx.x;
+}
 
 inline hipfftResult exec_r2c(hipfftHandle p, const double *in, void *out)
 {

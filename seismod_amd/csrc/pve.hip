@@ -53,14 +53,6 @@ struct PveStage {
     pstd::StageSrc<T> src;
 };
 
-template <typename T>
-__device__ __forceinline__ void rk(const PveStage<T> &a, size_t q, T d)
-{
-    const T s = a.ws[q];
-    if (a.set_t) a.wt[q] = s + a.a * d;
-    a.w[q] = (a.acc ? a.w[q] : s) + a.b * d;
-}
-
 // add_src_rk4 (src.c:77-112) for source s: p (Sf, Bulk), tau_xx (Sx, Bulk,
 // Bulk_s), tau_zz (Sz, Bulk, Bulk_s), tau_xz (Sxz)
 template <typename T>
@@ -86,52 +78,54 @@ __device__ __forceinline__ void pve_add_src(T *w, T *wt, size_t N, int s, int ns
 template <typename T, bool VTI>
 __global__ __launch_bounds__(256) void pve_stage(const PveStage<T> a)
 {
-    const unsigned n = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned n = pstd::cell_of_thread();
     if (n >= a.N) return;
     const size_t N = a.N;
     const int i = (int)(n / (unsigned)a.nz2), j = (int)(n % (unsigned)a.nz2);
+    // every input first (see RkCell)
     T d[L_NSET];
 #pragma unroll
-    for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.Ls[q], a.d[q * N + n], i, j, a.nx2, a.nz2, a.np);
+    for (int q = 0; q < L_NSET; ++q) d[q] = a.d[q * N + n];
     const T *m = a.mat;
+    const T rfi = m[M_RFI * N + n], mi = m[M_MI * N + n], irhoi = m[M_IRHOI * N + n];
+    const T rfj = m[M_RFJ * N + n], mj = m[M_MJ * N + n], irhoj = m[M_IRHOJ * N + n];
+    const T alpha = m[M_ALPHA * N + n], ts = m[M_TS * N + n], vphi = m[M_VPHI * N + n], M = m[M_M * N + n];
+    const T E = m[M_EM * N + n], Emu = m[M_EMU * N + n], muij = m[M_MUIJ * N + n];
+    const T alpha3 = VTI ? m[M_ALPHA3 * N + n] : alpha, c33 = VTI ? m[M_C33 * N + n] : E;
+    const T e = a.x[W_E * N + n];
+    pstd::RkCell<T, W_NF> rk;
+    rk.load(a.ws, a.w, a.acc, N, n);
+#pragma unroll
+    for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.Ls[q], d[q], i, j, a.nx2, a.nz2, a.np);
     // solid and fluid velocities on the interior nodes only (998-1005,
     // 1091-1098); elsewhere their rates stay 0
     const bool inner = i >= 1 && i < a.nx2 - 1 && j >= 1 && j < a.nz2 - 1;
-    T dvx = T(0), dqx = T(0), dvz = T(0), dqz = T(0);
+    T dl[W_NF];
+    dl[W_VX] = dl[W_QX] = dl[W_VZ] = dl[W_QZ] = T(0);
     if (inner) {
         const T t1 = d[L_DX_TXX] + d[L_DZ_TXZ];
-        dqx = (d[L_DX_P] + m[M_RFI * N + n] * t1) / m[M_MI * N + n];
-        dvx = m[M_IRHOI * N + n] * t1 - m[M_RFI * N + n] * dqx;
+        dl[W_QX] = (d[L_DX_P] + rfi * t1) / mi;
+        dl[W_VX] = irhoi * t1 - rfi * dl[W_QX];
         const T t2 = d[L_DX_TXZ] + d[L_DZ_TZZ];
-        dqz = (d[L_DZ_P] + m[M_RFJ * N + n] * t2) / m[M_MJ * N + n];
-        dvz = m[M_IRHOJ * N + n] * t2 - m[M_RFJ * N + n] * dqz;
+        dl[W_QZ] = (d[L_DZ_P] + rfj * t2) / mj;
+        dl[W_VZ] = irhoj * t2 - rfj * dl[W_QZ];
     }
-    rk(a, W_VX * N + n, dvx);
-    rk(a, W_QX * N + n, dqx);
-    rk(a, W_VZ * N + n, dvz);
-    rk(a, W_QZ * N + n, dqz);
     // epsilon = alpha (D_x^- v_x + D_z^- v_z) + D_x^- q_x + D_z^- q_z
     // (1100-1211); e, p, tau_xx, tau_zz (1213-1251)
-    const T alpha = m[M_ALPHA * N + n];
     T eps;
-    if (VTI) eps = alpha * d[L_DX_VX] + m[M_ALPHA3 * N + n] * d[L_DZ_VZ];
+    if (VTI) eps = alpha * d[L_DX_VX] + alpha3 * d[L_DZ_VZ];
     else eps = alpha * (d[L_DX_VX] + d[L_DZ_VZ]);
     eps += d[L_DX_QX];
     eps += d[L_DZ_QZ];
-    const T e = a.x[W_E * N + n];
-    rk(a, W_E * N + n, -m[M_TS * N + n] * (m[M_VPHI * N + n] * eps + e));
-    const T eps2 = m[M_M * N + n] * eps + e;
-    rk(a, W_P * N + n, -eps2);
-    const T E = m[M_EM * N + n], Emu = m[M_EMU * N + n];
-    if (VTI) {   // c11, c13, c33, alpha1, alpha3 (propagate.c:1864-1880)
-        rk(a, W_TXX * N + n, E * d[L_DX_VX] + Emu * d[L_DZ_VZ] + alpha * eps2);
-        rk(a, W_TZZ * N + n, Emu * d[L_DX_VX] + m[M_C33 * N + n] * d[L_DZ_VZ] + m[M_ALPHA3 * N + n] * eps2);
-    } else {
-        rk(a, W_TXX * N + n, E * d[L_DX_VX] + Emu * d[L_DZ_VZ] + alpha * eps2);
-        rk(a, W_TZZ * N + n, Emu * d[L_DX_VX] + E * d[L_DZ_VZ] + alpha * eps2);
-    }
+    dl[W_E] = -ts * (vphi * eps + e);
+    const T eps2 = M * eps + e;
+    dl[W_P] = -eps2;
+    // VTI: c11, c13, c33, alpha1, alpha3 (propagate.c:1864-1880)
+    dl[W_TXX] = E * d[L_DX_VX] + Emu * d[L_DZ_VZ] + alpha * eps2;
+    dl[W_TZZ] = Emu * d[L_DX_VX] + c33 * d[L_DZ_VZ] + alpha3 * eps2;
     // tau_xz (1259-1311)
-    rk(a, W_TXZ * N + n, m[M_MUIJ * N + n] * (d[L_DZ_VX] + d[L_DX_VZ]));
+    dl[W_TXZ] = muij * (d[L_DZ_VX] + d[L_DX_VZ]);
+    rk.store(a.w, a.wt, a.set_t, a.a, a.b, dl, N, n);
     for (int s = 0; s < a.src.n; ++s)
         if (a.src.cell[s] == (int)n)
             pve_add_src(a.w, a.wt, N, s, a.src.nsrc, a.src.tab, a.src.fct, a.src.dtw, a.src.dtt, a.src.it);
@@ -142,14 +136,16 @@ __global__ __launch_bounds__(256) void pve_stage(const PveStage<T> a)
 template <typename T>
 __global__ void pve_split(T *ws, const T *mat, unsigned N)
 {
-    const unsigned n = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned n = pstd::cell_of_thread();
     if (n >= N) return;
     const size_t NN = N;
-    const T qx = ws[W_QX * NN + n], qz = ws[W_QZ * NN + n];
-    ws[W_VX * NN + n] = ws[W_VX * NN + n] + mat[M_CVI * NN + n] * qx;
-    ws[W_VZ * NN + n] = ws[W_VZ * NN + n] + mat[M_CVJ * NN + n] * qz;
-    ws[W_QX * NN + n] = mat[M_CQI * NN + n] * qx;
-    ws[W_QZ * NN + n] = mat[M_CQJ * NN + n] * qz;
+    // every input before the first store
+    const T qx = ws[W_QX * NN + n], qz = ws[W_QZ * NN + n], vx = ws[W_VX * NN + n], vz = ws[W_VZ * NN + n];
+    const T cvi = mat[M_CVI * NN + n], cvj = mat[M_CVJ * NN + n], cqi = mat[M_CQI * NN + n], cqj = mat[M_CQJ * NN + n];
+    ws[W_VX * NN + n] = vx + cvi * qx;
+    ws[W_VZ * NN + n] = vz + cvj * qz;
+    ws[W_QX * NN + n] = cqi * qx;
+    ws[W_QZ * NN + n] = cqj * qz;
 }
 
 // all sources in order on one thread (more sources than the stage kernel
@@ -358,8 +354,8 @@ int stage(sm_pve *s, int tabs, bool last, const T *x, T a, T b, int set_t, int a
     L3(L_DZ_QZ, 1, np - 1, 1, T_B, K_K, T_B, K_K);
     L3(L_DZ_VX, 1, np, 1, T_BH, K_KH, T_BHE, K_KHE);
     L3(L_DX_VZ, 0, np, 0, T_BH, K_KH, T_BHE, K_KHE);
-    if (s->vti) pve_stage<T, true><<<pstd::blocks(N), 256, 0, st>>>(k);
-    else pve_stage<T, false><<<pstd::blocks(N), 256, 0, st>>>(k);
+    if (s->vti) pve_stage<T, true><<<pstd::cell_blocks(N), 256, 0, st>>>(k);
+    else pve_stage<T, false><<<pstd::cell_blocks(N), 256, 0, st>>>(k);
     return SM_OK;
 }
 
@@ -390,7 +386,7 @@ int run(sm_pve *s, size_t nsteps)
         const int64_t it = (int64_t)(s->step + k);
         if (s->timing) SM_HIP(hipEventRecord(ev[2 * k], st));
         std::swap(s->iw, s->iws);   // Ws = W, then the analytic step on it
-        pve_split<T><<<pstd::blocks(N), 256, 0, st>>>(STATE<T>(s, s->iws), (const T *)s->mat.ptr, (unsigned)N);
+        pve_split<T><<<pstd::cell_blocks(N), 256, 0, st>>>(STATE<T>(s, s->iws), (const T *)s->mat.ptr, (unsigned)N);
         for (int q = 0; q < 4; ++q) {
             const T *x = q == 0 ? STATE<T>(s, s->iws) : STATE<T>(s, s->iwt);
             int rc = stage<T>(s, stages[q].tabs, q == 3, x, stages[q].a, stages[q].b, q < 3 ? 1 : 0,

@@ -75,33 +75,32 @@ __device__ __forceinline__ void sh_add_src(T *w, T *wt, size_t N, int s, int nsr
 template <typename T>
 __global__ __launch_bounds__(256) void sh_stage(const ShStage<T> a)
 {
-    const unsigned n = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned n = pstd::cell_of_thread();
     if (n >= a.N) return;
     const unsigned N = a.N;
     const int i = (int)(n / (unsigned)a.nz2), j = (int)(n % (unsigned)a.nz2);
-    const T d0 = pstd::layer_fix(a.L[L_DX_TXY], a.d[n], i, j, a.nx2, a.nz2, a.np);
-    const T d1 = pstd::layer_fix(a.L[L_DZ_TYZ], a.d[N + n], i, j, a.nx2, a.nz2, a.np);
-    const T d2 = pstd::layer_fix(a.L[L_DZ_VY], a.d[2 * N + n], i, j, a.nx2, a.nz2, a.np);
-    const T d3 = pstd::layer_fix(a.L[L_DX_VY], a.d[3 * N + n], i, j, a.nx2, a.nz2, a.np);
-    const T *m = a.mat;
+    // every input first (see RkCell)
+    T d[L_NSET], m[M_NMAT];
+#pragma unroll
+    for (int q = 0; q < L_NSET; ++q) d[q] = a.d[(size_t)q * N + n];
+#pragma unroll
+    for (int q = 0; q < M_NMAT; ++q) m[q] = a.mat[(size_t)q * N + n];
+    const T e1 = a.x[(size_t)W_E1 * N + n], e2 = a.x[(size_t)W_E2 * N + n];
+    pstd::RkCell<T, W_NF> rk;
+    rk.load(a.ws, a.w, a.acc, N, n);
+#pragma unroll
+    for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.L[q], d[q], i, j, a.nx2, a.nz2, a.np);
     // v_y on the interior nodes only (propagate.c:2364-2374); elsewhere its
     // rate stays 0
     const bool inner = i >= 1 && i < a.nx2 - 1 && j >= 1 && j < a.nz2 - 1;
     T dl[W_NF];
-    dl[W_VY] = inner ? m[M_IRHO * N + n] * (d0 + d1) : T(0);
+    dl[W_VY] = inner ? m[M_IRHO] * (d[L_DX_TXY] + d[L_DZ_TYZ]) : T(0);
     // e' = (1/tau_s)((1 - 1/eta) D v - e);  tau' = c D v + c_0 e
-    const T e1 = a.x[W_E1 * N + n], e2 = a.x[W_E2 * N + n];
-    dl[W_E1] = m[M_TS1 * N + n] * (m[M_ETA1 * N + n] * d2 - e1);
-    dl[W_TYZ] = m[M_C44 * N + n] * d2 + m[M_C440 * N + n] * e1;
-    dl[W_E2] = m[M_TS2 * N + n] * (m[M_ETA2 * N + n] * d3 - e2);
-    dl[W_TXY] = m[M_C66 * N + n] * d3 + m[M_C660 * N + n] * e2;
-#pragma unroll
-    for (int c = 0; c < W_NF; ++c) {
-        const size_t q = (size_t)c * N + n;
-        const T s = a.ws[q];
-        if (a.set_t) a.wt[q] = s + a.a * dl[c];
-        a.w[q] = (a.acc ? a.w[q] : s) + a.b * dl[c];
-    }
+    dl[W_E1] = m[M_TS1] * (m[M_ETA1] * d[L_DZ_VY] - e1);
+    dl[W_TYZ] = m[M_C44] * d[L_DZ_VY] + m[M_C440] * e1;
+    dl[W_E2] = m[M_TS2] * (m[M_ETA2] * d[L_DX_VY] - e2);
+    dl[W_TXY] = m[M_C66] * d[L_DX_VY] + m[M_C660] * e2;
+    rk.store(a.w, a.wt, a.set_t, a.a, a.b, dl, N, n);
     for (int s = 0; s < a.src.n; ++s)
         if (a.src.cell[s] == (int)n)
             sh_add_src(a.w, a.wt, N, s, a.src.nsrc, a.src.tab, a.src.fct, a.src.dtw, a.src.dtt, a.src.it);
@@ -224,7 +223,7 @@ int stage(sm_sh *s, int tabs, bool last, const T *x, T a, T b, int set_t, int ac
     // columns (propagate.c:2410-2425, 2451-2455)
     k.L[L_DX_VY] = layer<T>(s->g, tabs, MEM<T>(s, 0, 1), MEM<T>(s, 1, 1), MEM<T>(s, 2, 1), 1, np, 0, T_BH,
                             K_KH, 1, T_BHE, K_KHE, r2x, r0x);
-    sh_stage<T><<<pstd::blocks(N), 256, 0, st>>>(k);
+    sh_stage<T><<<pstd::cell_blocks(N), 256, 0, st>>>(k);
     return SM_OK;
 }
 

@@ -75,51 +75,75 @@ __device__ __forceinline__ void ve_add_src(T *w, T *wt, size_t N, int s, int nsr
     if (typ == SM_SXZ) add(W_TXZ * N);
 }
 
-template <typename T>
-__device__ __forceinline__ void rk(const VeStage<T> &a, size_t q, T d)
-{
-    const T s = a.ws[q];
-    if (a.set_t) a.wt[q] = s + a.a * d;
-    a.w[q] = (a.acc ? a.w[q] : s) + a.b * d;
-}
-
-// propagate.c:1959-2278 from the eight derivatives on, then eq. (79)-(83)
-template <typename T>
+// propagate.c:1959-2278 from the eight derivatives on, then eq. (79)-(83);
+// LT: the number of dilatational mechanisms, 0 when only known at run time
+template <typename T, int LT>
 __global__ __launch_bounds__(256) void ve_stage(const VeStage<T> a)
 {
-    const unsigned n = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned n = pstd::cell_of_thread();
     if (n >= a.N) return;
     const size_t N = a.N;
     const int i = (int)(n / (unsigned)a.nz2), j = (int)(n % (unsigned)a.nz2);
-    T d[L_NSET];
+    const int L = LT ? LT : a.L;
+    constexpr int LA = LT ? LT : 1;
+    // every input first (see RkCell); the state components are the five
+    // fields, L dilatational variables, e2 and e3
+    T d[L_NSET], m[M_NFIX];
 #pragma unroll
-    for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.Ls[q], a.d[q * N + n], i, j, a.nx2, a.nz2, a.np);
-    const T *m = a.mat;
-    const int L = a.L;
-    // velocities on the interior nodes only (2044-2050, 2107-2112)
-    const bool inner = i >= 1 && i < a.nx2 - 1 && j >= 1 && j < a.nz2 - 1;
-    rk(a, W_VX * N + n, inner ? m[M_IRHOI * N + n] * (d[L_DX_TXX] + d[L_DZ_TXZ]) : T(0));
-    rk(a, W_VZ * N + n, inner ? m[M_IRHOJ * N + n] * (d[L_DX_TXZ] + d[L_DZ_TZZ]) : T(0));
-    // relaxation of the dilatation (2172-2180); the sum of tau_xx and
-    // tau_zz reads flat offset 6 N + n + k, as written (2190-2195)
-    const T t1 = d[L_DX_VX], t2 = d[L_DZ_VZ];
+    for (int q = 0; q < L_NSET; ++q) d[q] = a.d[q * N + n];
+#pragma unroll
+    for (int q = 0; q < M_NFIX; ++q) m[q] = a.mat[q * N + n];
+    // the relaxation sum of tau_xx and tau_zz reads flat offset 6 N + n + k,
+    // as written (2190-2195)
     T se = T(0);
     for (int k = 0; k < L; ++k) se += a.x[6 * N + n + k];
-    const T e2 = a.x[(5 + L) * N + n];
-    const T c550 = m[M_C550 * N + n], K0 = m[M_K0 * N + n];
-    rk(a, W_TXX * N + n, m[M_C11 * N + n] * t1 + m[M_C13 * N + n] * t2 + K0 * se + T(2) * c550 * e2);
-    rk(a, W_TZZ * N + n, m[M_C13 * N + n] * t1 + m[M_C33 * N + n] * t2 + K0 * se - T(2) * c550 * e2);
-    for (int k = 0; k < L; ++k) {
-        const T e1 = a.x[(W_E1 + k) * N + n];
-        rk(a, (W_E1 + k) * N + n,
-           m[(M_NFIX + L + k) * N + n] * (m[(M_NFIX + k) * N + n] * (t1 + t2) - e1));
+    const T e2 = a.x[(5 + L) * N + n], e3 = a.x[(6 + L) * N + n];
+    pstd::RkCell<T, W_E1> rk;
+    pstd::RkCell<T, 2> rk23;
+    pstd::RkCell<T, LA> rk1;
+    T e1[LA], ts1[LA], eta1[LA];
+    rk.load(a.ws, a.w, a.acc, N, n);
+    rk23.load(a.ws + (5 + L) * N, a.w + (5 + L) * N, a.acc, N, n);
+    if constexpr (LT > 0) {
+        rk1.load(a.ws + W_E1 * N, a.w + W_E1 * N, a.acc, N, n);
+#pragma unroll
+        for (int k = 0; k < LT; ++k) {
+            e1[k] = a.x[(W_E1 + k) * N + n];
+            eta1[k] = a.mat[(M_NFIX + k) * N + n];
+            ts1[k] = a.mat[(M_NFIX + L + k) * N + n];
+        }
     }
-    rk(a, (5 + L) * N + n, T(0.5) * m[M_TS2 * N + n] * (m[M_ETA2 * N + n] * (t1 + t2) - T(2) * e2));
+#pragma unroll
+    for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.Ls[q], d[q], i, j, a.nx2, a.nz2, a.np);
+    // velocities on the interior nodes only (2044-2050, 2107-2112)
+    const bool inner = i >= 1 && i < a.nx2 - 1 && j >= 1 && j < a.nz2 - 1;
+    T dl[W_E1], dl1[LA], dl23[2];
+    dl[W_VX] = inner ? m[M_IRHOI] * (d[L_DX_TXX] + d[L_DZ_TXZ]) : T(0);
+    dl[W_VZ] = inner ? m[M_IRHOJ] * (d[L_DX_TXZ] + d[L_DZ_TZZ]) : T(0);
+    // relaxation of the dilatation (2172-2180)
+    const T t1 = d[L_DX_VX], t2 = d[L_DZ_VZ];
+    const T c550 = m[M_C550], K0 = m[M_K0];
+    dl[W_TXX] = m[M_C11] * t1 + m[M_C13] * t2 + K0 * se + T(2) * c550 * e2;
+    dl[W_TZZ] = m[M_C13] * t1 + m[M_C33] * t2 + K0 * se - T(2) * c550 * e2;
+    dl23[0] = T(0.5) * m[M_TS2] * (m[M_ETA2] * (t1 + t2) - T(2) * e2);
     // e3 and tau_xz (2257-2263)
     const T u = d[L_DZ_VX] + d[L_DX_VZ];
-    const T e3 = a.x[(6 + L) * N + n];
-    rk(a, (6 + L) * N + n, m[M_TS2IJ * N + n] * (m[M_ETA2IJ * N + n] * u - e3));
-    rk(a, W_TXZ * N + n, m[M_C55 * N + n] * u);
+    dl23[1] = m[M_TS2IJ] * (m[M_ETA2IJ] * u - e3);
+    dl[W_TXZ] = m[M_C55] * u;
+    rk.store(a.w, a.wt, a.set_t, a.a, a.b, dl, N, n);
+    rk23.store(a.w + (5 + L) * N, a.wt + (5 + L) * N, a.set_t, a.a, a.b, dl23, N, n);
+    if constexpr (LT > 0) {
+#pragma unroll
+        for (int k = 0; k < LT; ++k) dl1[k] = ts1[k] * (eta1[k] * (t1 + t2) - e1[k]);
+        rk1.store(a.w + W_E1 * N, a.wt + W_E1 * N, a.set_t, a.a, a.b, dl1, N, n);
+    } else {
+        for (int k = 0; k < L; ++k) {
+            const size_t o = (W_E1 + k) * N;
+            rk1.load(a.ws + o, a.w + o, a.acc, N, n);
+            dl1[0] = a.mat[(M_NFIX + L + k) * N + n] * (a.mat[(M_NFIX + k) * N + n] * (t1 + t2) - a.x[o + n]);
+            rk1.store(a.w + o, a.wt + o, a.set_t, a.a, a.b, dl1, N, n);
+        }
+    }
     for (int s = 0; s < a.src.n; ++s)
         if (a.src.cell[s] == (int)n)
             ve_add_src(a.w, a.wt, N, s, a.src.nsrc, a.src.tab, a.src.fct, a.src.dtw, a.src.dtt, a.src.it);
@@ -242,7 +266,9 @@ int stage(sm_ve *s, int tabs, bool last, const T *x, T a, T b, int set_t, int ac
     L3(L_DZ_VZ, 1, np - 1, 1, T_B, K_K, T_B, K_K);
     L3(L_DZ_VX, 1, np, 1, T_BH, K_KH, T_BHE, K_KHE);
     L3(L_DX_VZ, 0, np, 0, T_BH, K_KH, T_BHE, K_KHE);
-    ve_stage<T><<<pstd::blocks(N), 256, 0, st>>>(k);
+    if (k.L == 1) ve_stage<T, 1><<<pstd::cell_blocks(N), 256, 0, st>>>(k);
+    else if (k.L == 2) ve_stage<T, 2><<<pstd::cell_blocks(N), 256, 0, st>>>(k);
+    else ve_stage<T, 0><<<pstd::cell_blocks(N), 256, 0, st>>>(k);
     return SM_OK;
 }
 
