@@ -156,8 +156,9 @@ typedef struct {
 #define SM_A3D_PAD64 4        /* fused kernels: device rows padded to a multiple
                                  of 64 cells; without
                                  the flag rows start on 128-byte lines when that
-                                 adds at most 5% (FP32) / 10% (16-bit) cells,
-                                 else they are padded to 8 cells */
+                                 adds at most 1/16 (FP32) / 1/7 (16-bit) of the
+                                 cells (5% / 10% with SM_A3D_SROUND), else they
+                                 are padded to 8 cells */
 #define SM_A3D_SROUND 2       /* BF16/FP16 storage: stochastic rounding of the
                                  stored values (deterministic pseudo-random
                                  bits from element index and step) instead

@@ -201,9 +201,14 @@ bool uses_fused(const sm_a3d_params &p)
 
 // device row pitch of the fused kernels: rows start on 128-byte cache
 // lines (a multiple of 32 cells in FP32, 64 in 16-bit storage; every
-// 64-cell wave access then covers whole lines) when that adds at most 5%
-// (FP32) or 10% (16-bit) cells, otherwise a multiple of 8 cells (16 bytes
-// of 16-bit storage; the TILE variants copy rows in 16-byte chunks).
+// 64-cell wave access then covers whole lines) when that adds at most 1/16
+// (FP32) or 1/7 (16-bit) of the cells, otherwise a multiple of 8 cells (16
+// bytes of 16-bit storage; the TILE variants copy rows in 16-byte chunks).
+// Measured, best launch of each: FP32 182 -> 192 cells (5.5%) 178 -> 163 us,
+// 296 -> 320 (8%) 308 -> 316; BF16 340 -> 384 (13%, 54 M cells, FP16
+// material) 409 -> 330, 220 -> 256 (16%) 120 -> 123.  Stochastic rounding
+// draws its bits by the device index, so there the limits stay 5% and 10%,
+// and a wider row must not take a grid past the 32-bit offsets.
 // SM_A3D_PAD64 forces a multiple of 64 cells.  The two-kernel paths keep
 // the reference layout.
 size_t row_pitch(size_t nz2, const sm_a3d_params &p)
@@ -214,6 +219,9 @@ size_t row_pitch(size_t nz2, const sm_a3d_params &p)
     const size_t line = wide ? 32 : 64;
     const size_t pl = (nz2 + line - 1) / line * line;
     if ((pl - nz2) * (wide ? 20 : 10) <= nz2) return pl;
+    const size_t cells = (p.nx + 2 * p.np) * (p.ny + 2 * p.np) * pl;
+    const bool fits = cells * 4 * (wide ? 4 : 2) <= 0xFFFFFF00u && cells * 8 <= 0xFFFFFF00u;
+    if (!(p.flags & SM_A3D_SROUND) && fits && (pl - nz2) * (wide ? 16 : 7) <= nz2) return pl;
     return (nz2 + 7) / 8 * 8;
 }
 

@@ -142,7 +142,7 @@ class A3dConfig:
     storage: str = "f32"
     naive: bool = False
     sround: bool = False      # BF16/FP16: stochastic rounding of stored values
-    pad64: bool = False       # rows always padded to 64 cells; else when <= 5% extra
+    pad64: bool = False       # rows always padded to 64 cells; else to cache lines where that costs little
     mat16: bool = False       # BF16/FP16: material as FP16 with power-of-two scales (tile variants)
 
     def params(self) -> L.A3dParams:
