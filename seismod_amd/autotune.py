@@ -83,7 +83,7 @@ def tune_a3d(sim, ctx, steps: int = 8, cache_file=None, candidates=None,
     nx2 = sim.cfg.nx + 2 * sim.cfg.np
     if candidates is None:
         candidates = [(tj, ch) for tj in (2, 4, 8) for ch in range(2, 17)
-                      if ch <= max(1, nx2 // 16)]
+                      if ch <= max(1, nx2 // 6)]
     best = None
     for v in variants:
         try:

@@ -693,17 +693,36 @@ int valid_chunks(int nx2, int want)
     return (nx2 + len - 1) / len;
 }
 
-// default launch shape: 4 waves per block; x chunks so that every resident
-// block slot gets about three items; persistent grid of resident size
+// default launch shape: 4 waves per block; persistent grid of resident size;
+// x chunks so that the items fill the resident slots once where that takes 4
+// chunks and more (cell kernel FP32, 120^3 cells: 5 chunks of 24 planes 31 us,
+// 20 of 6 18.5; 161 x 223 x 95: 6 chunks 35, 11 30, and 35 again at 13, where
+// the items pass the slots), else about three items a slot (260^3, tile: 2
+// chunks 264, 10 246)
 void default_launch(sm_a3d *s)
 {
     s->tj = 4;
     const int ntiles = z_tiles(s) * y_tiles(s);
     const int slots = resident_blocks(s, s->tj);
-    int nch = (3 * slots + ntiles - 1) / ntiles;
-    nch = std::min(nch, std::max(1, s->nx2 / 24));
+    const int once = slots / ntiles;
+    const int nch = once >= 4 ? std::min(once, std::max(1, s->nx2 / 6))
+                              : std::min((3 * slots + ntiles - 1) / ntiles, std::max(1, s->nx2 / 24));
     s->nchunks = valid_chunks(s->nx2, nch);
     s->nblocks = slots;
+}
+
+// default variant: the one-cell-a-lane kernel for FP32 grids whose two state
+// buffers and material stay in the 256 MB last-level cache beside the memory
+// variables of the layers, the tile kernel where they stream (best launch of
+// each: 161 x 223 x 95, 136 MB: cell 30 us, tile 40; 166^3, 183 MB: 39 and 47;
+// 182^3, 241 MB: 83 and 76; 192^3, 283 MB: 112 and 82).  16-bit storage
+// converts with every access and moves chunks at any size (BF16, cell and
+// tilesplit: 60^3 12.0 and 12.0, 120^3 27 and 24, 260^3 273 and 159, 340^3
+// 467 and 285).
+int default_variant(const sm_a3d *s)
+{
+    if (s->p.storage != SM_STORE_F32) return SM_A3D_TILE_SPLIT;
+    return s->nnp * (2 * 16 + 8) > ((size_t)224 << 20) ? SM_A3D_TILE : SM_A3D_CELL;
 }
 
 }  // namespace
@@ -779,7 +798,6 @@ int sm_a3d_create(sm_ctx *ctx, const sm_a3d_params *pp, const double *vp, const 
     const size_t nnp = s->nnp, pz = (size_t)s->pz;
     s->sr = (p.flags & SM_A3D_SROUND) && (p.storage == SM_STORE_BF16 || p.storage == SM_STORE_F16);
     s->m16 = (p.flags & SM_A3D_MAT16) != 0;
-    if (s->m16) s->variant = SM_A3D_TILE_SPLIT;   // the cell kernels read FP32 material
     // the fused kernel addresses the four state fields of one buffer and
     // the two material fields with 32-bit byte offsets
     if (s->fused && (4 * nnp * e > (size_t)0xFFFFFF00u || 2 * nnp * 4 > (size_t)0xFFFFFF00u)) {
@@ -793,7 +811,10 @@ int sm_a3d_create(sm_ctx *ctx, const sm_a3d_params *pp, const double *vp, const 
         if (hipGetDeviceProperties(&prop, ctx->device) == hipSuccess)
             s->cus = prop.multiProcessorCount;
     }
-    if (s->fused) default_launch(s);
+    if (s->fused) {
+        s->variant = default_variant(s);   // (the cell kernels read FP32 material)
+        default_launch(s);
+    }
     // one set (velocity or pressure) of x, y and z slab arrays
     const size_t slab_set = slab_cells(nx2, ny2, pz, p.np);
     int rc = SM_OK;

@@ -1,6 +1,7 @@
-"""GPU tests of the 3D solver's choices at creation: the row pitch, padded to
-cache lines or to 8 cells.  The choice only moves data around, so traces and
-fields are bit-identical to the other."""
+"""GPU tests of the 3D solver's choices at creation: the row pitch (padded to
+cache lines or to 8 cells) and the kernel variant (one cell a lane, or tiles
+where the wavefields leave the last-level cache).  Either choice only moves
+data and work around, so traces and fields are bit-identical to the other."""
 import numpy as np
 import pytest
 
@@ -32,3 +33,33 @@ def test_pitch_equals_forced_lines(ctx, nz2, storage, lines):
     b = run(ctx, d, storage, "cell", pad64=True)
     assert np.abs(a[0]).max() > 0
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+# below and above the line between the variants, few and many items a slot
+@pytest.mark.parametrize("shape,storage,variant", [
+    ((20, 9, 6, 3), "f32", "cell"), ((40, 150, 60, 4), "f32", "cell"),
+    ((178, 170, 176, 4), "f32", "tile"), ((20, 9, 6, 3), "bf16", "tilesplit"),
+    ((60, 150, 61, 4), "f16", "tilesplit")])
+def test_default_variant_equals_cell(ctx, shape, storage, variant):
+    from seismod_amd.solver import A3dConfig, Acoustic3D, source_functions
+    nx, ny, nz, np_ = shape
+    d = decks.a3d_deck(nx=nx, ny=ny, nz=nz, np_=np_, seed=5, nsteps=24)
+    c = d["cfg"]
+    got = []
+    for v in (None, "cell"):
+        s = Acoustic3D(ctx, A3dConfig(nx=nx, ny=ny, nz=nz, np=np_, dx=c["dx"], dy=c["dy"], dz=c["dz"],
+                                      dt=c["dt"], f0=c["f0"], vmax=c["vmax"], storage=storage),
+                       d["vp"], d["rho"])
+        if v is None:
+            assert s.variant() == variant
+        else:
+            s.set_variant(v)
+            s.set_launch(4, 1)
+        L, fct = source_functions(d["A"], d["f"], c["dt"])
+        s.set_sources(d["src_idx"], L, fct)
+        s.run(24)
+        got.append([s.field(k) for k in (8, 0, 1, 2)])
+        s.close()
+    assert np.abs(got[0][0]).max() > 0
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
