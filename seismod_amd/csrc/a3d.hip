@@ -340,16 +340,38 @@ float half_to_float(uint16_t h)
 }
 
 // state values on the host as double, scaled back to physical units
-int state_to_host(sm_a3d *s, const void *dev, size_t n, size_t stride_elems, size_t count,
-                  size_t pitch_elems, float scale, double *out)
+// rows of n elements, pitch apart, one after the other
+template <typename E>
+__global__ void a3d_pack(const E *src, E *dst, unsigned n, unsigned total, size_t pitch)
 {
-    // copies `count` rows of n values, rows `pitch_elems` apart on the device
+    const unsigned q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < total) dst[q] = src[(size_t)(q / n) * pitch + q % n];
+}
+
+// copies `count` rows of n values, rows `pitch_elems` apart on the device.
+// A strided copy to the host goes row by row (400 rows of 340 BF16 cells: 2.8
+// ms, as long as 8 steps), so the fused path packs the rows into the half of
+// its state that the next step overwrites, every cell of it, and copies them
+// in one piece (0.07 ms); the one-half layouts have no such space.
+int state_to_host(sm_a3d *s, const void *dev, size_t n, size_t count, size_t pitch_elems, float scale, double *out)
+{
     const size_t e = s->elt;
     std::vector<unsigned char> tmp(n * count * e);
-    SM_HIP(hipMemcpy2DAsync(tmp.data(), n * e, dev, pitch_elems * e, n * e, count,
-                            hipMemcpyDeviceToHost, s->ctx->stream));
-    SM_HIP(hipStreamSynchronize(s->ctx->stream));
-    (void)stride_elems;
+    hipStream_t st = s->ctx->stream;
+    if (s->fused && count > 1 && pitch_elems != n) {
+        void *half = s->fields[1 - s->cur].ptr;
+        const unsigned tot = (unsigned)(n * count), nb = (tot + 255) / 256;
+        if (e == 4) a3d_pack<<<nb, 256, 0, st>>>((const uint32_t *)dev, (uint32_t *)half, (unsigned)n, tot, pitch_elems);
+        else a3d_pack<<<nb, 256, 0, st>>>((const uint16_t *)dev, (uint16_t *)half, (unsigned)n, tot, pitch_elems);
+        SM_HIP(hipGetLastError());
+        dev = half;
+        pitch_elems = n;
+    }
+    if (pitch_elems == n)
+        SM_HIP(hipMemcpyAsync(tmp.data(), dev, n * count * e, hipMemcpyDeviceToHost, st));
+    else
+        SM_HIP(hipMemcpy2DAsync(tmp.data(), n * e, dev, pitch_elems * e, n * e, count, hipMemcpyDeviceToHost, st));
+    SM_HIP(hipStreamSynchronize(st));
     const size_t tot = n * count;
     switch (s->p.storage) {
     case SM_STORE_F64:
@@ -1143,7 +1165,7 @@ int sm_a3d_get_field(sm_a3d *s, int comp, double *out)
     SM_CHECK(slot >= 0, SM_ERR_ARG, "sm_a3d_get_field: component %d", comp);
     SM_CHECK(set_device(s->ctx) == SM_OK, SM_ERR_HIP, "hipSetDevice failed");
     const char *src = (const char *)s->fields[s->cur].ptr + slot * s->nnp * s->elt;
-    return state_to_host(s, src, s->nz2, 0, (size_t)s->nx2 * s->ny2, s->pz,
+    return state_to_host(s, src, s->nz2, (size_t)s->nx2 * s->ny2, s->pz,
                          slot == 0 ? s->sP : s->sV, out);
 }
 
@@ -1156,7 +1178,7 @@ int sm_a3d_get_slice_xz(sm_a3d *s, int comp, size_t iy, double *out)
     SM_CHECK(set_device(s->ctx) == SM_OK, SM_ERR_HIP, "hipSetDevice failed");
     const char *base = (const char *)s->fields[s->cur].ptr + slot * s->nnp * s->elt +
                        iy * (size_t)s->pz * s->elt;
-    return state_to_host(s, base, s->nz2, 0, s->nx2, (size_t)s->ny2 * s->pz,
+    return state_to_host(s, base, s->nz2, s->nx2, (size_t)s->ny2 * s->pz,
                          slot == 0 ? s->sP : s->sV, out);
 }
 

@@ -1,7 +1,8 @@
 """GPU tests of the 3D solver's choices at creation: the row pitch (padded to
 cache lines or to 8 cells) and the kernel variant (one cell a lane, or tiles
 where the wavefields leave the last-level cache).  Either choice only moves
-data and work around, so traces and fields are bit-identical to the other."""
+data and work around, so traces and fields are bit-identical to the other.
+And of reading slices and fields between runs."""
 import numpy as np
 import pytest
 
@@ -61,5 +62,38 @@ def test_default_variant_equals_cell(ctx, shape, storage, variant):
         got.append([s.field(k) for k in (8, 0, 1, 2)])
         s.close()
     assert np.abs(got[0][0]).max() > 0
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+# padded and whole rows, every element size, with and without a second half
+@pytest.mark.parametrize("nx,ny,nz,np_,storage", [
+    (9, 7, 13, 3, "f32"), (9, 7, 58, 3, "f32"), (9, 7, 13, 3, "bf16"), (3, 6, 61, 0, "f16"),
+    (3, 3, 9, 0, "f32"), (40, 33, 51, 2, "bf16"), (9, 7, 13, 3, "f64")])
+def test_slices_between_runs(ctx, nx, ny, nz, np_, storage):
+    """Slices and fields taken between runs agree with each other and leave
+    the run as it is without them."""
+    from seismod_amd.solver import A3dConfig, Acoustic3D, source_functions
+    d = decks.a3d_deck(nx=nx, ny=ny, nz=nz, np_=np_, seed=3, nsteps=30)
+    c = d["cfg"]
+    got = []
+    for look in (False, True):
+        s = Acoustic3D(ctx, A3dConfig(nx=nx, ny=ny, nz=nz, np=np_, dx=c["dx"], dy=c["dy"], dz=c["dz"],
+                                      dt=c["dt"], f0=c["f0"], vmax=c["vmax"], storage=storage),
+                       d["vp"], d["rho"])
+        L, fct = source_functions(d["A"], d["f"], c["dt"])
+        s.set_sources(d["src_idx"], L, fct)
+        s.set_receivers(d["rec_idx"], d["rec_comp"], 30)
+        for n in (1, 12, 2, 15):
+            if look:
+                for comp in (8, 1):
+                    f = s.field(comp)
+                    for iy in (0, f.shape[1] - 1):
+                        assert np.array_equal(s.slice_xz(comp, iy), f[:, iy, :])
+                    assert np.array_equal(s.field(comp), f)
+            s.run(n)
+        got.append([s.traces(0, 30)] + [s.field(k) for k in (8, 0, 1, 2)])
+        s.close()
+    assert np.abs(got[0][1]).max() > 0
     for a, b in zip(*got):
         assert np.array_equal(a, b)
