@@ -127,16 +127,18 @@ __device__ __forceinline__ T layer_fix(const Layer<T> &L, T d, int i, int j, int
 // after a store waits its turn, and a cell's inputs then arrive one memory
 // round trip after the other.  (Bound by memory: an SH stage of 1040^2 FP32
 // moves its 138 MB at 5.6 TB/s.  Measured per launch, loads in place, all
-// loads first, and with the cells of cell_of_thread: sh_stage 1040^2 FP32
-// 27.9, 26.7, 24.6 us; ve_stage 469 x 363 FP64 22.7, 21.2, 18.8; pve_stage
-// 1040^2 FP32 52.4, 51.9, 49.4, 640 x 480 FP64 VTI 36.0, 37.0, 33.1.)
+// loads first, with the cells of cell_of_thread, and without s in the last
+// stage: sh_stage 1040^2 FP32 27.9, 26.7, 24.6, 23.5 us; ve_stage 469 x 363
+// FP64 22.7, 21.2, 18.8, 18.5; pve_stage 1040^2 FP32 52.4, 51.9, 49.4, 45.9,
+// 640 x 480 FP64 VTI 36.0, 37.0, 33.1, 32.3.)
 template <typename T, int NF>
 struct RkCell {
     T s[NF], w[NF];
-    __device__ __forceinline__ void load(const T *ws, const T *wa, int acc, size_t N, size_t n)
+    // (the last stage, which accumulates and sets no wt, has no use for s)
+    __device__ __forceinline__ void load(const T *ws, const T *wa, int acc, int set_t, size_t N, size_t n)
     {
 #pragma unroll
-        for (int c = 0; c < NF; ++c) s[c] = ws[c * N + n];
+        for (int c = 0; c < NF; ++c) s[c] = set_t || !acc ? ws[c * N + n] : T(0);
 #pragma unroll
         for (int c = 0; c < NF; ++c) w[c] = acc ? wa[c * N + n] : s[c];
     }

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void pve_stage(const PveStage<T> a)
     const T alpha3 = VTI ? m[M_ALPHA3 * N + n] : alpha, c33 = VTI ? m[M_C33 * N + n] : E;
     const T e = a.x[W_E * N + n];
     pstd::RkCell<T, W_NF> rk;
-    rk.load(a.ws, a.w, a.acc, N, n);
+    rk.load(a.ws, a.w, a.acc, a.set_t, N, n);
 #pragma unroll
     for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.Ls[q], d[q], i, j, a.nx2, a.nz2, a.np);
     // solid and fluid velocities on the interior nodes only (998-1005,

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void sh_stage(const ShStage<T> a)
     for (int q = 0; q < M_NMAT; ++q) m[q] = a.mat[(size_t)q * N + n];
     const T e1 = a.x[(size_t)W_E1 * N + n], e2 = a.x[(size_t)W_E2 * N + n];
     pstd::RkCell<T, W_NF> rk;
-    rk.load(a.ws, a.w, a.acc, N, n);
+    rk.load(a.ws, a.w, a.acc, a.set_t, N, n);
 #pragma unroll
     for (int q = 0; q < L_NSET; ++q) d[q] = pstd::layer_fix(a.L[q], d[q], i, j, a.nx2, a.nz2, a.np);
     // v_y on the interior nodes only (propagate.c:2364-2374); elsewhere its

@@ -102,10 +102,10 @@ __global__ __launch_bounds__(256) void ve_stage(const VeStage<T> a)
     pstd::RkCell<T, 2> rk23;
     pstd::RkCell<T, LA> rk1;
     T e1[LA], ts1[LA], eta1[LA];
-    rk.load(a.ws, a.w, a.acc, N, n);
-    rk23.load(a.ws + (5 + L) * N, a.w + (5 + L) * N, a.acc, N, n);
+    rk.load(a.ws, a.w, a.acc, a.set_t, N, n);
+    rk23.load(a.ws + (5 + L) * N, a.w + (5 + L) * N, a.acc, a.set_t, N, n);
     if constexpr (LT > 0) {
-        rk1.load(a.ws + W_E1 * N, a.w + W_E1 * N, a.acc, N, n);
+        rk1.load(a.ws + W_E1 * N, a.w + W_E1 * N, a.acc, a.set_t, N, n);
 #pragma unroll
         for (int k = 0; k < LT; ++k) {
             e1[k] = a.x[(W_E1 + k) * N + n];
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void ve_stage(const VeStage<T> a)
     } else {
         for (int k = 0; k < L; ++k) {
             const size_t o = (W_E1 + k) * N;
-            rk1.load(a.ws + o, a.w + o, a.acc, N, n);
+            rk1.load(a.ws + o, a.w + o, a.acc, a.set_t, N, n);
             dl1[0] = a.mat[(M_NFIX + L + k) * N + n] * (a.mat[(M_NFIX + k) * N + n] * (t1 + t2) - a.x[o + n]);
             rk1.store(a.w + o, a.wt + o, a.set_t, a.a, a.b, dl1, N, n);
         }
