@@ -272,7 +272,7 @@ def main_cyl(args) -> None:
         sys.exit(1)
     nx2, nz2 = shot.vp.shape
     elt = 4 if args.storage == "f32" else 8
-    alg_b = synth.algorithmic_bytes_cyl(nx2, nz2, shot.np, elt=elt)
+    alg_b = synth.algorithmic_bytes_cyl(nx2, nz2, shot.np, elt=elt, torsional=shot.mode != 0)
     avg_ms = kms / max(timed, 1)
     achieved = alg_b * shot.cells / (avg_ms * 1e-3) / 1e9
     line = {

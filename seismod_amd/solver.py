@@ -406,8 +406,9 @@ class Elastic2D:
 
 
 class E2dBatch:
-    """Runs many Elastic2D shots (FP32 fused) together: one launch per time
-    step over all shots still running, replayed from hipGraphs."""
+    """Runs many Elastic2D shots (FP32 fused) together: launches of several
+    time steps over all shots still running (one step per launch, replayed
+    from hipGraphs, where a grid has no second split buffer)."""
 
     def __init__(self, ctx: Context, graph_steps: int = 32):
         self.ctx = ctx

@@ -331,17 +331,20 @@ def cyl_borehole_shot(nx: int = 1000, nz: int = 4000, np_: int = 20, dr: float =
                    rec_comp=np.array([r[1] for r in rec], dtype=np.intc))
 
 
-def algorithmic_bytes_cyl(nx2: int, nz2: int, np_: int, elt: int = 4) -> float:
+def algorithmic_bytes_cyl(nx2: int, nz2: int, np_: int, elt: int = 4, torsional: bool = True) -> float:
     """Minimal HBM bytes per padded cell per step of the e_cyl_iso update.
 
     The nine fields (v_r, v_theta, v_z and six stresses) read and written
     once and the eight material arrays (lambda, lambda+2mu, three mu and
     three buoyancy averages) read once: 26 values; plus the CPML memory
     variables, read and written once where they exist (18 arrays over the
-    np+1 outer rows, 6 over the 2np+1 slots of every row)."""
+    np+1 outer rows, 6 over the 2np+1 slots of every row).  Without the
+    torsional fields (mode 0, no Ft source): six fields, five material
+    arrays, 8 and 4 memory variables."""
     cells = nx2 * nz2
-    mem = (18 * (np_ + 1) * nz2 + 6 * nx2 * (2 * np_ + 1)) if np_ else 0
-    return elt * (26.0 + 2.0 * mem / cells)
+    values, r, z = (26.0, 18, 6) if torsional else (17.0, 8, 4)
+    mem = (r * (np_ + 1) * nz2 + z * nx2 * (2 * np_ + 1)) if np_ else 0
+    return elt * (values + 2.0 * mem / cells)
 
 
 @dataclass
