@@ -436,9 +436,16 @@ size_t sm_cyl_bytes_needed(const sm_cyl_params *p, size_t nrec, size_t max_steps
 typedef struct sm_sh sm_sh;
 /* flags of sm_sh_params and sm_ve_params (no counterpart in the reference):
  * take every derivative through hipFFT even where the hand-written
- * LDS transforms apply (axis lengths whose factors are 2, 3, 5, 7, 11, 13);
- * both give the same results to rounding */
+ * LDS transforms apply (sm_pstd_plan); both give the same results to
+ * rounding */
 #define SM_PSTD_HIPFFT 1
+/* How the pseudo-spectral solvers take the derivatives along an axis of n
+ * points (layers included) in SM_STORE_F32 or SM_STORE_F64 (no counterpart
+ * in the reference): *points, the length of the hand-written transform (n, or
+ * the padded length of a line with a prime factor above 13), 0 for hipFFT;
+ * *rounds, in how many rounds a workgroup takes its longest pass.  Needs no
+ * device. */
+int sm_pstd_plan(size_t n, int storage, int *points, int *rounds);
 typedef struct {
     size_t nx, nz;            /* interior nodes (struct grid) */
     size_t np;                /* CPML layers on every side (nl); forced to 0

@@ -171,6 +171,7 @@ _SIGS = {
     "sm_cyl_reset": (C.c_int, [C.c_void_p]),
     "sm_cyl_device_bytes": (C.c_int, [C.c_void_p, _size_p]),
     "sm_cyl_bytes_needed": (C.c_size_t, [C.POINTER(CylParams), C.c_size_t, C.c_size_t]),
+    "sm_pstd_plan": (C.c_int, [C.c_size_t, C.c_int, _int_p, _int_p]),
     "sm_sh_create": (C.c_int, [C.c_void_p, C.POINTER(ShParams), _dbl_p, _dbl_p, _dbl_p, _dbl_p, _dbl_p,
                                C.POINTER(C.c_void_p)]),
     "sm_sh_destroy": (C.c_int, [C.c_void_p]),

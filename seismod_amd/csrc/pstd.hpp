@@ -18,11 +18,13 @@
 //   z (unit stride): real-to-complex and complex-to-real transforms.
 // Results equal the real-transform derivatives to rounding.
 //
-// Axes whose transforms fit a workgroup's LDS skip hipFFT: one pstd_dfft
+// Axes whose length has a plan (fft_plan) skip hipFFT: one pstd_dfft
 // launch (pstd_fft.hpp) takes every derivative of a stage along both axes,
 // with one read and one write per value instead of six (forward transform,
-// multiplier pass, inverse transform).  hipFFT remains for longer axes and
-// on request (SM_PSTD_HIPFFT).
+// multiplier pass, inverse transform).  hipFFT remains on request
+// (SM_PSTD_HIPFFT) and for lengths without a plan: factors above 13 and more
+// than 2048 points, or more than 3584 points (FP64 1792) and no radices that
+// 512 threads take in one round.
 //
 // CPML (pml.c:1959-2106): per stage (fp1, fp23, fp4) and axis the rows b,
 // c at nodes, bh, ch at inner half nodes, bH, cH at outer half nodes; the
@@ -255,6 +257,12 @@ struct DJob {
     bool fwd;
 };
 
+// pstd_rounds.hip: the kernel of lines in several rounds, and its launch
+template <typename T>
+const void *rounds_kernel();
+template <typename T>
+void rounds_launch(unsigned grid, unsigned nt, size_t lds, hipStream_t st, const DfftArgs<T> &ax, const DfftArgs<T> &az);
+
 // pairs per thread (V) and groups of V pairs per workgroup (P) of a launch of
 // nx derivatives along x and nz along z
 struct FftShape {
@@ -278,9 +286,11 @@ inline FftShape fft_shape(const Grid &g, size_t elt, int nx, int nz)
     // (1040^2 FP32, 4 derivatives: 19.0 against 23.3 us), one pair halves
     // the serial chain and wins where the grid leaves compute units idle
     // (200^2: 6.6 against 8.2 us).  FP64 values of two pairs take all 256
-    // registers (1040^2: 44 against 40 us).
+    // registers (1040^2: 44 against 40 us), and so do loops over items
+    // (3000^2 FP32, a step: 1809 against 1531 us).
     FftShape s;
-    s.V = elt == 4 && fits(2, 1) && blocks(2, 1) >= 2 * g.cus ? 2 : 1;
+    const bool loop = (nx && g.fft[0].loop) || (nz && g.fft[1].loop);
+    s.V = elt == 4 && !loop && fits(2, 1) && blocks(2, 1) >= 2 * g.cus ? 2 : 1;
     // Workgroups are much alike, so the launch takes the time of the compute
     // unit with the most of them: P that leaves them evenly spread, and of
     // two alike the larger, whose x accesses cover more of a cache line
@@ -344,7 +354,10 @@ DfftArgs<T> dfft_args(const Grid &g, int axis, const T *x, T *d, const DJob *job
 }
 
 // the derivatives xj[0..nx) along x and zj[0..nz) along z of the fields
-// of x into d: one launch for the axes with own transforms
+// of x into d: one launch for the axes with own transforms, or one each when
+// only one of them loops (its workgroups have eight waves and more registers,
+// and the short lines of the other axis would hold a compute unit each: a step
+// of 256 x 3000 FP32 214 us in one launch, 177 in two)
 template <typename T>
 int deriv_xz(Grid &g, const T *x, T *d, const DJob *xj, int nx, const DJob *zj, int nz)
 {
@@ -360,6 +373,10 @@ int deriv_xz(Grid &g, const T *x, T *d, const DJob *xj, int nx, const DJob *zj, 
         count[ax] = 0;
     }
     if (count[0] + count[1] == 0) return SM_OK;
+    if (count[0] && count[1] && g.fft[0].loop != g.fft[1].loop) {
+        int rc = deriv_xz<T>(g, x, d, xj, nx, zj, 0);
+        return rc == SM_OK ? deriv_xz<T>(g, x, d, xj, 0, zj, nz) : rc;
+    }
     DfftArgs<T> a[2] = {};
     size_t lds = 0;
     unsigned nt = 64;
@@ -373,7 +390,9 @@ int deriv_xz(Grid &g, const T *x, T *d, const DJob *xj, int nx, const DJob *zj, 
         nt = std::max(nt, t);
     }
     const unsigned grid = (unsigned)((a[0].nblocks + 7) / 8 + (a[1].nblocks + 7) / 8) * 8;
-    const bool pad = (count[0] && g.fft[0].m != g.fft[0].n) || (count[1] && g.fft[1].m != g.fft[1].n);
+    auto any = [&](auto f) { return (count[0] && f(g.fft[0])) || (count[1] && f(g.fft[1])); };
+    const bool loop = any([](const FftPlan &p) { return p.loop; });
+    const bool pad = any([](const FftPlan &p) { return p.m != p.n; });
     hipStream_t st = g.ctx->stream;
     if constexpr (sizeof(T) == 4) {
         if (sh.V == 2) {
@@ -382,7 +401,8 @@ int deriv_xz(Grid &g, const T *x, T *d, const DJob *xj, int nx, const DJob *zj, 
             return SM_OK;
         }
     }
-    if (pad) pstd_dfft<T, 1, true><<<grid, nt, lds, st>>>(a[0], a[1]);
+    if (loop) rounds_launch<T>(grid, nt, lds, st, a[0], a[1]);
+    else if (pad) pstd_dfft<T, 1, true><<<grid, nt, lds, st>>>(a[0], a[1]);
     else pstd_dfft<T, 1, false><<<grid, nt, lds, st>>>(a[0], a[1]);
     return SM_OK;
 }
@@ -500,14 +520,17 @@ inline size_t kmul_bytes(size_t nx2, size_t nz2, size_t elt)
     return 2 * (std::max(nx2, nx2 / 2 + 1) + nz2 / 2 + 1) * 2 * elt;
 }
 
-// LDS one workgroup of transforms may take: all 160 KiB of a compute unit
-// when the runtime grants it
+// LDS one workgroup of transforms may take: all of a compute unit's when the
+// runtime grants it
+constexpr size_t FFT_LDS = 160 * 1024;
 inline size_t fft_lds_limit(size_t elt)
 {
-    const int want = 160 * 1024;
-    const void *k8[] = {(const void *)pstd_dfft<double, 1, false>, (const void *)pstd_dfft<double, 1, true>};
+    const int want = (int)FFT_LDS;
+    const void *k8[] = {(const void *)pstd_dfft<double, 1, false>, (const void *)pstd_dfft<double, 1, true>,
+                        rounds_kernel<double>()};
     const void *k4[] = {(const void *)pstd_dfft<float, 1, false>, (const void *)pstd_dfft<float, 1, true>,
-                        (const void *)pstd_dfft<float, 2, false>, (const void *)pstd_dfft<float, 2, true>};
+                        (const void *)pstd_dfft<float, 2, false>, (const void *)pstd_dfft<float, 2, true>,
+                        rounds_kernel<float>()};
     bool ok = true;
     auto grant = [&](const void *k) {
         ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, want) == hipSuccess;
@@ -589,7 +612,7 @@ inline int init(Grid &g, sm_ctx *ctx, size_t nx2, size_t nz2, size_t np, size_t 
         const size_t n = ax == 0 ? nx2 : nz2;
         const double d = ax == 0 ? dx : dz;
         FftPlan &f = g.fft[ax];
-        if (!fft_plan((int)n, f) || fft_lds(f, 1, 1, elt) > lds_limit) continue;
+        if (!fft_plan((int)n, elt, f) || fft_lds(f, 1, 1, elt) > lds_limit) continue;
         std::vector<double> fm;
         for (double sgn : {1.0, -1.0}) {
             const std::vector<double> h = fft_spectrum(f, d, sgn);
@@ -635,7 +658,7 @@ inline size_t grid_bytes(size_t nx2, size_t nz2, size_t np, size_t elt)
     size_t own = 0;
     for (size_t n : {nx2, nz2}) {
         FftPlan f;
-        if (fft_plan((int)n, f)) own += ((size_t)std::max(f.tsz, 1) + 2 * (size_t)f.m) * 2 * elt;
+        if (fft_plan((int)n, elt, f)) own += ((size_t)std::max(f.tsz, 1) + 2 * (size_t)f.m) * 2 * elt;
     }
     return spec_bytes(nx2, nz2, elt) + kmul_bytes(nx2, nz2, elt) + table_bytes(np, elt) + own;
 }

@@ -260,11 +260,15 @@ struct FftPlan {
     int S[FFT_MAXPASS] = {};        // distance of a butterfly's elements
     int toff[FFT_MAXPASS] = {}, tsz = 0;   // twiddles of pass q at toff[q], (t - 1) S + j
     double cost = 0;                // per element
+    bool loop = false;              // a pass takes its butterflies in several rounds
 };
 
-// the cheapest radices of m; false when m has a factor above 13 or needs
-// fewer than two or more than FFT_MAXPASS passes
-inline bool fft_radices(int m, FftPlan &p)
+constexpr int FFT_THREADS = 512;    // largest workgroup: 256 registers a thread
+
+// the cheapest radices of m, none below `least`; false when m has a factor
+// above 13, no such radices, or needs fewer than two or more than
+// FFT_MAXPASS passes
+inline bool fft_radices(int m, int least, FftPlan &p)
 {
     p.nr = 0;
     p.cost = 1e30;
@@ -279,7 +283,7 @@ inline bool fft_radices(int m, FftPlan &p)
             return;
         }
         if (k == FFT_MAXPASS) return;
-        for (int r = std::min(most, left); r >= 2; --r)
+        for (int r = std::min(most, left); r >= least; --r)
             if (left % r == 0) {
                 cur[k] = r;
                 self(self, left / r, r, k + 1, c + fft_cost(r) + FFT_PASS);
@@ -307,46 +311,65 @@ inline void fft_layout(FftPlan &p)
     }
 }
 
-constexpr int FFT_THREADS = 512;    // largest workgroup: 256 registers a thread
 // threads of a workgroup: every pass takes its butterflies in one round
+// unless the plan loops
 inline int fft_threads(const FftPlan &p, int P)
 {
     int most = 0;
     for (int q = 0; q < p.nr; ++q) most = std::max(most, P * (p.m / p.R[q]));
+    if (p.loop) most = std::min(most, FFT_THREADS);
     return (most + 63) / 64 * 64;
 }
 
-// plan of the derivative of n points; false when no hand-written transform
-// takes this length.  The derivative is a circular convolution with a real
-// kernel of n points, so a length with other factors runs as a linear one:
+// plan of the derivative of n points in values of elt bytes; false when no
+// hand-written transform takes this length.
+//
+// First choice are the cheapest radices with which FFT_THREADS threads take
+// every pass in one round: of 2000 points, none below 4.  A line of at most
+// FFT_LOOP bytes that has none takes the cheapest of all and loops (1617 to
+// 3402 points in FP32, 1617 in FP64).  A step of the SH solver, FP32, this
+// loop against hipFFT: 256 x 3000 177 and 301 us, 3000 x 256 183 and 425,
+// 256 x 2662 184 and 297, 3000^2 1531 and 3556.  Longer lines stay with
+// hipFFT: 256 x 4000 343 us, 391 in one round of 1024 threads.
+//
+// The derivative is a circular convolution with a real kernel of n points, so
+// a length with other factors runs as a linear one:
 // lines padded with zeros to any m >= 2 n - 1 that the radices make, and the
 // kernel's spectrum over m points as the multiplier: twice the work of a
 // length that the radices make (1039^2 against 1040^2, 8 FP32 derivatives:
 // 77.6 and 36.2 us), a quarter of hipFFT's chirp transforms and their copy
-// passes (469 x 363, FP64, a P-SV stage: 45 against 230 us).
-inline bool fft_plan(int n, FftPlan &p)
+// passes (469 x 363, FP64, a P-SV stage: 45 against 230 us).  One round of
+// FFT_THREADS threads takes m up to 4096, n up to 2048.
+constexpr size_t FFT_LOOP = 28 * 1024;
+inline bool fft_plan(int n, size_t elt, FftPlan &p)
 {
+    auto one_round = [](int m) { return std::max(2, (m + FFT_THREADS - 1) / FFT_THREADS); };
     p = FftPlan();
     if (n < 2) return false;
-    if (fft_radices(n, p)) {
-        p.m = n;
-    } else {
-        FftPlan best;
+    p.m = n;
+    bool ok = fft_radices(n, one_round(n), p);
+    if (!ok && 2 * (size_t)n * elt <= FFT_LOOP) ok = p.loop = fft_radices(n, 2, p);
+    if (!ok) {
         double cost = 1e30;
         for (int m = 2 * n - 1; m <= 2 * n + n / 4 + 16; ++m) {
             FftPlan f;
-            if (!fft_radices(m, f) || f.cost * m >= cost) continue;
-            f.m = m;
-            if (fft_threads(f, 1) > FFT_THREADS) continue;
+            if (!fft_radices(m, one_round(m), f) || f.cost * m >= cost) continue;
+            ok = true;
             cost = f.cost * m;
-            best = f;
+            p = f;
+            p.m = m;
         }
-        if (best.nr == 0) return false;
-        p = best;
     }
     p.n = n;
-    fft_layout(p);
-    return fft_threads(p, 1) <= FFT_THREADS;
+    if (ok) fft_layout(p);
+    return ok;
+}
+// rounds of the longest pass of one group of lines
+inline int fft_rounds(const FftPlan &p)
+{
+    int most = 0;
+    for (int q = 0; q < p.nr; ++q) most = std::max(most, p.m / p.R[q]);
+    return (most + FFT_THREADS - 1) / FFT_THREADS;
 }
 
 // whole-spectrum multiplier of the forward (sgn 1) or backward (-1)
@@ -652,12 +675,60 @@ __device__ __forceinline__ void dft_group(Cx<T> (&v)[V][R])
     for (int g = 0; g < V; ++g) dft<T, R>(v[g]);
 }
 
+#define PSTD_RADIX(r, CALL)                                                                         \
+    switch (r) {                                                                                    \
+    case 2: { constexpr int R = 2; CALL; break; }                                                   \
+    case 3: { constexpr int R = 3; CALL; break; }                                                   \
+    case 4: { constexpr int R = 4; CALL; break; }                                                   \
+    case 5: { constexpr int R = 5; CALL; break; }                                                   \
+    case 6: { constexpr int R = 6; CALL; break; }                                                   \
+    case 7: { constexpr int R = 7; CALL; break; }                                                   \
+    case 8: { constexpr int R = 8; CALL; break; }                                                   \
+    case 9: { constexpr int R = 9; CALL; break; }                                                   \
+    case 10: { constexpr int R = 10; CALL; break; }                                                 \
+    case 11: { constexpr int R = 11; CALL; break; }                                                 \
+    case 12: { constexpr int R = 12; CALL; break; }                                                 \
+    case 13: { constexpr int R = 13; CALL; break; }                                                 \
+    case 14: { constexpr int R = 14; CALL; break; }                                                 \
+    case 15: { constexpr int R = 15; CALL; break; }                                                 \
+    default: { constexpr int R = 16; CALL; break; }                                                 \
+    }
+
+// The passes and the kernel: one item a thread, or, for pstd_rounds.hip, loops
+// over the items of a pass.  (Two texts of one source in two translation
+// units and not a template: any form of loop in the one-round kernels, even
+// one the compiler removes, and the loop kernels' code between theirs moved
+// their steps by up to 5%: 256 x 1296 FP64 156 and 165 us.)
+#ifdef PSTD_ROUNDS
+#define PSTD_ITEMS for (uint32_t l = threadIdx.x; l < items; l += blockDim.x)
+namespace rounds {
+#else
+#define PSTD_ITEMS const uint32_t l = threadIdx.x; if (l < items)
+#endif
+
 // first pass: global memory -> LDS
 template <typename T, int V, int R, int AX, bool PAD>
 __device__ __forceinline__ void pass_first(const DfftArgs<T> &a, const FftIO<T, V> &io)
 {
     const uint32_t S = a.S[0], items = a.nb[0] << a.lP;
     const uint32_t lst = S + a.pad * divm(S, a.mL);
+#ifdef PSTD_ROUNDS
+    for (int q = threadIdx.x; q < a.tsz; q += blockDim.x) io.tw[q] = a.tw[q];
+    __syncthreads();
+    PSTD_ITEMS {
+        uint32_t p, j;
+        outer_item<T, AX>(a, l, p, j);
+        Cx<T> v[V][R];
+#pragma unroll
+        for (int g = 0; g < V; ++g)
+#pragma unroll
+            for (int t = 0; t < R; ++t) v[g][t] = {T(0), T(0)};
+        load_lines<T, V, R, AX, PAD>(a, io, (int)p, j, v);
+        dft_group<T, V, R>(v);
+        twiddle<T, V, R>(io.tw + j, S, v);
+        lds_store<T, V, R>(io.A + p * a.ls + lds_at(a, j), lst, v);
+    }
+#else
     const uint32_t l = threadIdx.x;
     uint32_t p = 0, j = 0;
     Cx<T> v[V][R];
@@ -677,6 +748,7 @@ __device__ __forceinline__ void pass_first(const DfftArgs<T> &a, const FftIO<T, 
         twiddle<T, V, R>(io.tw + j, S, v);
         lds_store<T, V, R>(io.A + p * a.ls + lds_at(a, j), lst, v);
     }
+#endif
 }
 
 // a pass between the first and the middle one, forward or transposed
@@ -685,8 +757,7 @@ __device__ __forceinline__ void pass_inner(const DfftArgs<T> &a, const FftIO<T, 
 {
     const uint32_t S = a.S[q], nb = a.nb[q], items = nb << a.lP;
     const uint32_t lst = S + a.pad * divm(S, a.mL);
-    const uint32_t l = threadIdx.x;
-    if (l < items) {
+    PSTD_ITEMS {
         const uint32_t p = divm(l, a.mN[q]), b = l - p * nb;
         const uint32_t blk = divm(b, a.mS[q]), j = b - blk * S;
         Elem<T, V> *s = io.A + p * a.ls + lds_at(a, blk * S * R + j);
@@ -706,8 +777,7 @@ __device__ __forceinline__ void pass_mid(const DfftArgs<T> &a, const FftIO<T, V>
 {
     const int q = a.nr - 1;
     const uint32_t nb = a.nb[q], items = nb << a.lP;
-    const uint32_t l = threadIdx.x;
-    if (l < items) {
+    PSTD_ITEMS {
         const uint32_t p = divm(l, a.mN[q]), b = l - p * nb;
         Cx<T> h[R], v[V][R];
 #pragma unroll
@@ -733,8 +803,7 @@ __device__ __forceinline__ void pass_last(const DfftArgs<T> &a, const FftIO<T, V
 {
     const uint32_t S = a.S[0], items = a.nb[0] << a.lP;
     const uint32_t lst = S + a.pad * divm(S, a.mL);
-    const uint32_t l = threadIdx.x;
-    if (l < items) {
+    PSTD_ITEMS {
         uint32_t p, j;
         outer_item<T, AX>(a, l, p, j);
         Cx<T> v[V][R];
@@ -745,24 +814,6 @@ __device__ __forceinline__ void pass_last(const DfftArgs<T> &a, const FftIO<T, V
     }
 }
 
-#define PSTD_RADIX(r, CALL)                                                                         \
-    switch (r) {                                                                                    \
-    case 2: { constexpr int R = 2; CALL; break; }                                                   \
-    case 3: { constexpr int R = 3; CALL; break; }                                                   \
-    case 4: { constexpr int R = 4; CALL; break; }                                                   \
-    case 5: { constexpr int R = 5; CALL; break; }                                                   \
-    case 6: { constexpr int R = 6; CALL; break; }                                                   \
-    case 7: { constexpr int R = 7; CALL; break; }                                                   \
-    case 8: { constexpr int R = 8; CALL; break; }                                                   \
-    case 9: { constexpr int R = 9; CALL; break; }                                                   \
-    case 10: { constexpr int R = 10; CALL; break; }                                                 \
-    case 11: { constexpr int R = 11; CALL; break; }                                                 \
-    case 12: { constexpr int R = 12; CALL; break; }                                                 \
-    case 13: { constexpr int R = 13; CALL; break; }                                                 \
-    case 14: { constexpr int R = 14; CALL; break; }                                                 \
-    case 15: { constexpr int R = 15; CALL; break; }                                                 \
-    default: { constexpr int R = 16; CALL; break; }                                                 \
-    }
 // the derivative of the lines of tile b: AX 1 z (unit stride, row pairs
 // r, r + 1), AX 0 x (stride nz2, column pairs c, c + 1); a missing partner
 // reads as 0 and is not written
@@ -794,8 +845,8 @@ __device__ __forceinline__ void dfft_body(const DfftArgs<T> &a, int b)
 }
 
 // the derivatives of a stage along x (ax) and z (az) in one grid (either may
-// have none); PAD: a line is shorter than its transform.  Every XCD takes a range of consecutive x tiles (adjacent
-// columns share cache lines) and then a range of z tiles: the x tiles move
+// have none); PAD: a line is shorter than its transform.  Every XCD takes a
+// range of consecutive x tiles (adjacent columns share cache lines) and then a range of z tiles: the x tiles move
 // more cache lines and take longer, so giving half of the XCDs only x tiles
 // would leave the others waiting.
 template <typename T, int V, bool PAD>
@@ -809,6 +860,11 @@ __global__ __launch_bounds__(FFT_THREADS) void pstd_dfft(const DfftArgs<T> ax, c
         if (xcd * pz + i - px < az.nblocks) dfft_body<T, V, 1, PAD>(az, xcd * pz + i - px);
     }
 }
+
+#undef PSTD_ITEMS
+#ifdef PSTD_ROUNDS
+}  // namespace rounds
+#endif
 
 // LDS elements of one group of pairs: the padded line, spread so that the P
 // groups that lanes touch at one position lie on different banks (a row of

@@ -367,6 +367,20 @@ bool material(size_t nx2, size_t nz2, const double *mu, const double *rho, const
 
 extern "C" {
 
+int sm_pstd_plan(size_t n, int storage, int *points, int *rounds)
+{
+    SM_CHECK(points && rounds, SM_ERR_ARG, "sm_pstd_plan: NULL argument");
+    SM_CHECK(storage == SM_STORE_F32 || storage == SM_STORE_F64, SM_ERR_ARG, "sm_pstd_plan: storage %d not supported",
+             storage);
+    SM_CHECK(n >= 1 && n < (1u << 30), SM_ERR_ARG, "sm_pstd_plan: %zu points", n);
+    const size_t elt = storage == SM_STORE_F64 ? 8 : 4;
+    pstd::FftPlan f;
+    const bool own = pstd::fft_plan((int)n, elt, f) && pstd::fft_lds(f, 1, 1, elt) <= pstd::FFT_LDS;
+    *points = own ? f.m : 0;
+    *rounds = own ? pstd::fft_rounds(f) : 0;
+    return SM_OK;
+}
+
 size_t sm_sh_bytes_needed(const sm_sh_params *p, size_t nrec, size_t max_steps)
 {
     if (!p || (p->storage != SM_STORE_F64 && p->storage != SM_STORE_F32)) return 0;

@@ -36,6 +36,15 @@ def ricker_length(f: float, dt: float) -> int:
     return int(lib.sm_ricker_length(f, dt))
 
 
+def pstd_plan(n: int, storage: str) -> tuple[int, int]:
+    """How the pseudo-spectral solvers differentiate along an axis of n points
+    (layers included): the points of the hand-written transform (0: hipFFT) and
+    the rounds of its longest pass."""
+    points, rounds = C.c_int(), C.c_int()
+    check(lib.sm_pstd_plan(n, _STORAGE[storage], C.byref(points), C.byref(rounds)), "sm_pstd_plan")
+    return points.value, rounds.value
+
+
 def source_functions(A, f, dt: float) -> tuple[np.ndarray, np.ndarray]:
     """compute_src_fct (src.c:43-65): returns (lengths, concatenated fct)."""
     A = _f64(np.atleast_1d(A))
