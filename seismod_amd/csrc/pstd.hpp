@@ -81,6 +81,7 @@ struct Grid {
     bool own[2] = {false, false};
     FftPlan fft[2];
     int cus = 256;                  // compute units of the device
+    size_t lds = 0;                 // bytes of LDS a workgroup may take
     sm_dbuf tw[2], fmul[2];
 };
 
@@ -278,7 +279,8 @@ inline FftShape fft_shape(const Grid &g, size_t elt, int nx, int nz)
     };
     auto fits = [&](int V, int P) {
         for (int ax = 0; ax < 2; ++ax)
-            if (count[ax] && (fft_lds(g.fft[ax], V, P, elt) > 81920 || fft_threads(g.fft[ax], P) > FFT_THREADS))
+            if (count[ax] && (fft_lds(g.fft[ax], V, P, elt) > std::min<size_t>(g.lds, 81920) ||
+                              fft_threads(g.fft[ax], P) > FFT_THREADS))
                 return false;
         return true;
     };
@@ -605,14 +607,14 @@ inline int init(Grid &g, sm_ctx *ctx, size_t nx2, size_t nz2, size_t np, size_t 
     }
     // hand-written transforms: twiddles and the multipliers over the whole
     // spectrum in the order of the middle pass
-    const size_t lds_limit = own ? fft_lds_limit(elt) : 0;
+    g.lds = own ? fft_lds_limit(elt) : 0;
     if (hipDeviceGetAttribute(&g.cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess || g.cus < 1)
         g.cus = 256;
     for (int ax = 0; ax < 2 && rc == SM_OK && own; ++ax) {
         const size_t n = ax == 0 ? nx2 : nz2;
         const double d = ax == 0 ? dx : dz;
         FftPlan &f = g.fft[ax];
-        if (!fft_plan((int)n, elt, f) || fft_lds(f, 1, 1, elt) > lds_limit) continue;
+        if (!fft_plan((int)n, elt, f) || fft_lds(f, 1, 1, elt) > g.lds) continue;
         std::vector<double> fm;
         for (double sgn : {1.0, -1.0}) {
             const std::vector<double> h = fft_spectrum(f, d, sgn);
