@@ -263,6 +263,10 @@ typedef struct {
 
 #define SM_E2D_NAIVE 1        /* FP32 with the reference-order two-kernel
                                  step instead of the fused one */
+#define SM_E2D_ONESTEP 2      /* fused FP32: one step a launch, in the form of
+                                 sm_e2d_set_launch and sm_e2d_set_variant, and
+                                 no second split buffer (24 bytes a padded cell
+                                 less); identical results */
 
 /* Build a solver from interior vp, vs, rho (nx*nz each, read_model_e,
  * io_utils.c:892-947): Lame constants and staggered averages
@@ -296,12 +300,16 @@ int sm_e2d_device_bytes(const sm_e2d *s, size_t *bytes);
  * below 2 GiB (about 4730^2 padded cells) */
 size_t sm_e2d_bytes_needed(const sm_e2d_params *p, size_t nrec, size_t max_steps);
 
+/* Whether runs of two steps and more take several steps a launch: *on 1
+ * unless SM_E2D_ONESTEP, SM_E2D_NAIVE, FP64 or a grid above about 4230^2
+ * padded cells (no counterpart in the reference) */
+int sm_e2d_get_multistep(const sm_e2d *s, int *on);
 /* Launch shape of the fused FP32 step where a launch takes one step (runs of
- * one step, grids above about 4230^2 padded cells, the allocation-free
- * batches; longer runs advance several steps per launch and choose their
- * own shape; no counterpart in the reference): x rows each wavefront marches
- * over, and steps per captured hipGraph (0 or 1: plain launches).  Results
- * do not depend on either. */
+ * one step, solvers without multistep, batches with such a shot, the
+ * allocation-free batches; other runs advance several steps per launch and
+ * choose their own shape; no counterpart in the reference): x rows each
+ * wavefront marches over, and steps per captured hipGraph (0 or 1: plain
+ * launches).  Results do not depend on either. */
 int sm_e2d_set_launch(sm_e2d *s, int rows_per_chunk, int graph_steps);
 int sm_e2d_get_launch(const sm_e2d *s, int *rows_per_chunk, int *graph_steps);
 /* Kernel form of the one-step launch (no counterpart in the reference):

@@ -31,6 +31,8 @@ SM_A3D_TILE_SPLIT = 6
 SM_A3D_TILE_NT = 7
 SM_A3D_TILE_SPLIT_NT = 8
 SM_PROBE_NT = 16
+SM_E2D_NAIVE = 1
+SM_E2D_ONESTEP = 2
 SM_E2D_ROWS = 0
 SM_E2D_STAGED = 1
 SM_PROBE_TILES = 32
@@ -143,6 +145,7 @@ _SIGS = {
     "sm_e2d_set_variant": (C.c_int, [C.c_void_p, C.c_int]),
     "sm_e2d_get_variant": (C.c_int, [C.c_void_p, _int_p]),
     "sm_e2d_batch_set_variant": (C.c_int, [C.c_void_p, C.c_int]),
+    "sm_e2d_get_multistep": (C.c_int, [C.c_void_p, _int_p]),
     "sm_e2d_get_launch": (C.c_int, [C.c_void_p, _int_p, _int_p]),
     "sm_e2d_set_timing": (C.c_int, [C.c_void_p, C.c_int]),
     "sm_e2d_get_timing": (C.c_int, [C.c_void_p, _dbl_p, _size_p]),

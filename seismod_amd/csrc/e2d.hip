@@ -382,10 +382,18 @@ static bool e2d_fused_fits(size_t N)
 }
 
 // floats of the fused solver's state: a second split buffer, for several
-// steps per launch, as long as the whole stays below the same bound (24
-// bytes more per cell; larger grids run a launch a step as before)
-static bool e2d_tiles(size_t N) { return (2 * E2_NSTATE + 2 * E2_NSPLIT) * N * 4 < (1ull << 31); }
-static size_t e2d_state_floats(size_t N) { return (2 * E2_NSTATE + (e2d_tiles(N) ? 2 : 1) * E2_NSPLIT) * N; }
+// steps per launch (24 bytes more per cell), unless the caller asks for one
+// step a launch or the whole passes the same bound.  (No kernel needs that:
+// each buffer has a resource of its own.  Grids of 17.9 to 22.4 M cells keep
+// the launch a step they are tested with.)
+static bool e2d_tiles(size_t N, int flags)
+{
+    return !(flags & SM_E2D_ONESTEP) && (2 * E2_NSTATE + 2 * E2_NSPLIT) * N * 4 < (1ull << 31);
+}
+static size_t e2d_state_floats(size_t N, int flags)
+{
+    return (2 * E2_NSTATE + (e2d_tiles(N, flags) ? 2 : 1) * E2_NSPLIT) * N;
+}
 
 size_t sm_e2d_bytes_needed(const sm_e2d_params *p, size_t nrec, size_t max_steps)
 {
@@ -394,7 +402,7 @@ size_t sm_e2d_bytes_needed(const sm_e2d_params *p, size_t nrec, size_t max_steps
     const size_t NX = p->nx + 2 * p->npml, NZ = p->nz + 2 * p->npml, N = NX * NZ;
     if (p->storage == SM_STORE_F32 && !(p->flags & SM_E2D_NAIVE)) {
         if (!e2d_fused_fits(N)) return 0;   // sm_e2d_create refuses the grid
-        return 4 * (e2d_state_floats(N) + E2_NMAT * N + 4 * (NX + NZ) + nrec * max_steps) +
+        return 4 * (e2d_state_floats(N, p->flags) + E2_NMAT * N + 4 * (NX + NZ) + nrec * max_steps) +
                16 * nrec + 4096;
     }
     return e * (20 * N + 4 * (NX + NZ) + nrec * max_steps) + 16 * nrec;
@@ -411,7 +419,7 @@ int sm_e2d_create(sm_ctx *ctx, const sm_e2d_params *pp, const double *vp, const 
     SM_CHECK(p.h > 0 && p.dt > 0, SM_ERR_ARG, "sm_e2d_create: h and dt must be > 0");
     SM_CHECK(p.storage == SM_STORE_F32 || p.storage == SM_STORE_F64, SM_ERR_ARG,
              "sm_e2d_create: storage %d not supported", p.storage);
-    SM_CHECK((p.flags & ~SM_E2D_NAIVE) == 0, SM_ERR_ARG, "sm_e2d_create: unknown flags %#x", p.flags);
+    SM_CHECK((p.flags & ~(SM_E2D_NAIVE | SM_E2D_ONESTEP)) == 0, SM_ERR_ARG, "sm_e2d_create: unknown flags %#x", p.flags);
     const size_t nx = p.nx, nz = p.nz, np = p.npml, n = nx * nz;
     const size_t NX = nx + 2 * np, NZ = nz + 2 * np, N = NX * NZ;
     SM_CHECK(NX < (1u << 20) && NZ < (1u << 20), SM_ERR_ARG, "sm_e2d_create: grid too large");
@@ -556,8 +564,8 @@ int sm_e2d_create(sm_ctx *ctx, const sm_e2d_params *pp, const double *vp, const 
         SM_CHECK(e2d_fused_fits(N), SM_ERR_ARG,
                  "sm_e2d_create: padded grid %zux%zu too large for the fused FP32 kernel "
                  "(state and split fields must stay below 2 GiB; use SM_E2D_NAIVE or FP64)", NX, NZ);
-        s->tiles = e2d_tiles(N);
-        rc = dalloc(s->fields, e2d_state_floats(N) * 4);
+        s->tiles = e2d_tiles(N, p.flags);
+        rc = dalloc(s->fields, e2d_state_floats(N, p.flags) * 4);
         // 16 floats past the last material array: the staged kernel's
         // 16-byte chunks of the last row may extend into them
         if (rc == SM_OK) rc = dalloc(s->mat, (E2_NMAT * N + 16) * 4);
@@ -848,6 +856,13 @@ int sm_e2d_get_variant(const sm_e2d *s, int *variant)
 {
     SM_CHECK(s && variant, SM_ERR_ARG, "sm_e2d_get_variant: NULL argument");
     *variant = s->fused ? s->variant : -1;
+    return SM_OK;
+}
+
+int sm_e2d_get_multistep(const sm_e2d *s, int *on)
+{
+    SM_CHECK(s && on, SM_ERR_ARG, "sm_e2d_get_multistep: NULL argument");
+    *on = s->tiles ? 1 : 0;
     return SM_OK;
 }
 

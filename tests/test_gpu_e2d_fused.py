@@ -1,8 +1,11 @@
 """GPU tests of the fused FP32 2D elastic step and of shot batches.
 
-The fused kernel's arithmetic per cell does not depend on the launch shape
-(rows per chunk, graph replay), on how a run is split, or on which other
+The fused kernels' arithmetic per cell does not depend on the form (several
+steps a launch, or one step as rows or staged), on the launch shape (rows per
+chunk, graph replay), on how a run is split, or on which other
 shots share the launch, so all of those must give bit-identical results.
+Forms and shapes of the one-step launch are tested on solvers that take no
+other (one_step), against the several steps a launch of an ordinary one.
 Against the FP64 oracle it is held to a relative-L2 tolerance, and against
 the reference-order FP32 kernels to a tighter one (same precision, only the
 folding of dt/h and the PML coefficients differ).
@@ -25,12 +28,13 @@ def rel_l2(a, b):
     return float(np.linalg.norm(a - b) / (den if den > 0 else 1.0))
 
 
-def make(ctx, d, naive=False, launch=None):
+def make(ctx, d, naive=False, launch=None, one_step=False):
     from seismod_amd.solver import E2dConfig, Elastic2D, source_functions
     c = d["cfg"]
     cfg = E2dConfig(nx=c["nx"], nz=c["nz"], npml=c["npml"], h=c["h"], dt=c["dt"], storage="f32",
-                    q1_compat=c.get("q1_compat", True), naive=naive)
+                    q1_compat=c.get("q1_compat", True), naive=naive, one_step=one_step)
     s = Elastic2D(ctx, cfg, d["vp"], d["vs"], d["rho"])
+    assert s.multistep() == (not naive and not one_step)
     if launch is not None:
         s.set_launch(*launch)
     lengths, fct = source_functions(d["A"], d["f"], c["dt"])
@@ -88,6 +92,15 @@ def test_fused_vs_oracle(ctx, case):
     assert e_tr < TOL_ORACLE and e_f < TOL_ORACLE
 
 
+def test_one_step_memory(ctx):
+    """Without the second split buffer a solver holds 24 bytes a cell less,
+    and bytes_needed says so."""
+    d = deck(nx=60, nz=70, npml=8, seed=11, nsteps=20)
+    a, b = make(ctx, d), make(ctx, d, one_step=True)
+    assert a.device_bytes() - b.device_bytes() == 24 * 76 * 86
+    assert a.cfg.bytes_needed(12, 20) - b.cfg.bytes_needed(12, 20) == 24 * 76 * 86
+
+
 @pytest.mark.parametrize("case", CASES[:6], ids=ids)
 def test_fused_vs_naive_fp32(ctx, case):
     d = deck(**case)
@@ -102,19 +115,20 @@ def test_fused_vs_naive_fp32(ctx, case):
 @pytest.mark.parametrize("launch", [(1, 0), (2, 4), (3, 1), (7, 32), (64, 8), (4096, 0)])
 def test_launch_shape_invariance(ctx, launch):
     d = deck(nx=60, nz=70, npml=8, seed=11, nsteps=90)
-    ref = make(ctx, d, launch=(8, 0))
+    ref = make(ctx, d)
     ref.run(d["nsteps"])
-    s = make(ctx, d, launch=launch)
+    s = make(ctx, d, launch=launch, one_step=True)
     s.run(d["nsteps"])
     (t0, f0), (t1, f1) = outputs(ref), outputs(s)
     assert np.array_equal(t0, t1) and np.array_equal(f0, f1)
 
 
-def test_run_splitting_and_reset(ctx):
+@pytest.mark.parametrize("one_step", [False, True])
+def test_run_splitting_and_reset(ctx, one_step):
     d = deck(nx=50, nz=40, npml=5, seed=12, nsteps=100)
-    a = make(ctx, d, launch=(4, 8))
+    a = make(ctx, d)
     a.run(100)
-    b = make(ctx, d, launch=(4, 8))
+    b = make(ctx, d, launch=(4, 8), one_step=one_step)
     for n in (1, 30, 17, 52):
         b.run(n)
     (ta, fa), (tb, fb) = outputs(a), outputs(b)
@@ -226,25 +240,27 @@ def test_batch_argument_errors(ctx):
 def test_staged_equals_rows(ctx, case, launch):
     """The staged kernel (rows of the next step as 16-byte chunks through
     LDS) computes the same values as the per-lane form, for every chunk
-    length, grid width (rows not 16-byte aligned) and PML thickness."""
+    length, grid width (rows not 16-byte aligned) and PML thickness; and both
+    the same as several steps a launch."""
     d = deck(**case)
-    a = make(ctx, d, launch=launch)
-    a.run(d["nsteps"])
-    ra = outputs(a)
-    a.close()
-    b = make(ctx, d, launch=launch)
-    b.set_variant("staged")
-    assert b.variant() == "staged"
-    b.run(d["nsteps"])
-    rb = outputs(b)
-    b.close()
-    assert np.abs(ra[0]).max() > 0
-    assert np.array_equal(ra[0], rb[0]) and np.array_equal(ra[1], rb[1])
+    t = make(ctx, d)
+    t.run(d["nsteps"])
+    rt = outputs(t)
+    t.close()
+    assert np.abs(rt[0]).max() > 0
+    for variant in ("rows", "staged"):
+        b = make(ctx, d, launch=launch, one_step=True)
+        b.set_variant(variant)
+        assert b.variant() == variant
+        b.run(d["nsteps"])
+        rb = outputs(b)
+        b.close()
+        assert np.array_equal(rt[0], rb[0]) and np.array_equal(rt[1], rb[1]), variant
 
 
 def test_staged_batch_equals_alone(ctx):
     """A staged batch of shots of different sizes and step counts equals
-    each shot run alone with the per-lane kernel."""
+    each shot run alone."""
     from seismod_amd.solver import E2dBatch
     specs = [dict(nx=37, nz=23, npml=4, seed=21, nsteps=60), dict(nx=16, nz=70, npml=3, seed=22, nsteps=45),
              dict(nx=51, nz=130, npml=7, seed=23, nsteps=80), dict(nx=9, nz=9, npml=1, seed=24, nsteps=30)]
@@ -255,10 +271,11 @@ def test_staged_batch_equals_alone(ctx):
         s.run(d["nsteps"])
         alone.append(outputs(s))
         s.close()
-    sims = [make(ctx, d, launch=(2, 0)) for d in ds]
+    sims = [make(ctx, d, launch=(2, 0), one_step=True) for d in ds]
     b = E2dBatch(ctx, graph_steps=8)
     b.set_variant("staged")
     b.run(sims, [d["nsteps"] for d in ds])
+    assert b.graphs()[1] > 0
     b.close()
     for s, (tr, f) in zip(sims, alone):
         got = outputs(s)

@@ -1,7 +1,7 @@
 """Several FP32 2D steps per launch (halos recomputed in registers) against
 the same steps run one launch each: the expressions are the same, so the
 results are compared bit for bit.  A run of one step always takes the
-one-step kernel.
+one-step kernel (its forms and launch shapes: test_gpu_e2d_fused.py).
 
 Grids around the tile's edges (owned rows and columns depend on the number of
 steps of a launch), layers thinner and thicker than a wave's rows, step
