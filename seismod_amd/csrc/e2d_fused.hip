@@ -762,24 +762,35 @@ int grid_blocks(int nitems)
 
 E2dRunner::~E2dRunner()
 {
-    drop_graphs();
+    destroy_graphs();   // (the owner has waited for its stream)
     if (table_) (void)hipFree(table_);
     if (base_) (void)hipFree(base_);
 }
 
-void E2dRunner::drop_graphs()
+void E2dRunner::destroy_graphs()
 {
     for (auto &kv : graphs_) (void)hipGraphExecDestroy(kv.second.exec);
     graphs_.clear();
 }
 
+// the graphs of an earlier table; replays of them (an earlier group's) may
+// still be queued on the stream
+int E2dRunner::drop_graphs(hipStream_t st)
+{
+    if (graphs_.empty()) return SM_OK;
+    SM_HIP(hipStreamSynchronize(st));
+    destroy_graphs();
+    return SM_OK;
+}
+
 size_t E2dRunner::device_bytes() const { return table_cap_ + (base_ ? 256 : 0); }
 
-int E2dRunner::ensure(size_t bytes)
+int E2dRunner::ensure(size_t bytes, hipStream_t st)
 {
     if (!base_) SM_HIP(hipMalloc((void **)&base_, 256));
     if (bytes <= table_cap_) return SM_OK;
-    drop_graphs();
+    int rc = drop_graphs(st);
+    if (rc != SM_OK) return rc;
     if (table_) SM_HIP(hipFree(table_));
     table_ = nullptr;
     table_cap_ = 0;
@@ -969,9 +980,10 @@ int E2dRunner::run_tiles(std::vector<E2dShot> &shots, hipStream_t st)
     for (size_t i = 0; i < n; ++i)
         for (int q = pref[i]; q < pref[i + 1]; ++q) bs[q] = (int)i;
     // (captured graphs read the table's memory)
-    drop_graphs();
+    int rc = drop_graphs(st);
+    if (rc != SM_OK) return rc;
     last_tab_bytes_ = 0;
-    int rc = ensure(host.size());
+    rc = ensure(host.size(), st);
     if (rc != SM_OK) return rc;
     SM_HIP(hipMemcpyAsync(table_, host.data(), host.size(), hipMemcpyHostToDevice, st));
     SM_HIP(hipStreamSynchronize(st));
@@ -1024,11 +1036,13 @@ int E2dRunner::run(std::vector<E2dShot> shots, hipStream_t st, int graph_steps)
     int rc = plan(shots, pref, host, tab_bytes);
     if (rc != SM_OK || shots.empty()) return rc;
     tab_bytes_ = tab_bytes;
-    if (host.size() > table_cap_ || tab_bytes_ != last_tab_bytes_ || staged != last_staged_)
-        drop_graphs();
+    if (host.size() > table_cap_ || tab_bytes_ != last_tab_bytes_ || staged != last_staged_) {
+        rc = drop_graphs(st);
+        if (rc != SM_OK) return rc;
+    }
     last_tab_bytes_ = tab_bytes_;
     last_staged_ = staged;
-    rc = ensure(host.size());
+    rc = ensure(host.size(), st);
     if (rc != SM_OK) return rc;
     // the table lives in device memory read by the kernels of this run;
     // waiting for the copy keeps the host buffer's lifetime simple

@@ -122,7 +122,7 @@ public:
 private:
     void launch_step(int nb, hipStream_t st, const E2dShot *tab, const int *bshot, int nitems,
                      const int *base, int k);
-    int ensure(size_t bytes);
+    int ensure(size_t bytes, hipStream_t st);
     int run_tiles(std::vector<E2dShot> &shots, hipStream_t st);
     E2dTile tile_;
     int cus_ = 0;
@@ -132,7 +132,8 @@ private:
     int launch_all(const std::vector<E2dShot> &shots, const std::vector<int> &pref,
                    const void *table, size_t tab_bytes, hipStream_t st, int graph_steps,
                    size_t *count);
-    void drop_graphs();
+    void destroy_graphs();
+    int drop_graphs(hipStream_t st);
     void *table_ = nullptr;     // shot descriptors, then the block -> shot map
     size_t table_cap_ = 0;      // bytes
     size_t tab_bytes_ = 0, last_tab_bytes_ = 0;

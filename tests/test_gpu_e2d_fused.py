@@ -140,7 +140,8 @@ def test_run_splitting_and_reset(ctx, one_step):
     assert np.array_equal(ta, tc) and np.array_equal(fa, fc)
 
 
-def test_batch_equals_alone(ctx):
+@pytest.mark.parametrize("one_step", [False, True])
+def test_batch_equals_alone(ctx, one_step):
     """Shots of different sizes, step counts and starting steps, batched,
     give the same bits as each run alone."""
     from seismod_amd.solver import E2dBatch
@@ -158,7 +159,7 @@ def test_batch_equals_alone(ctx):
         s.run(d["nsteps"])
         alone.append(outputs(s))
         s.close()
-    shots = [make(ctx, d, launch=(5, 0)) for d in dks]
+    shots = [make(ctx, d, launch=(5, 0), one_step=one_step) for d in dks]
     # two shots start ahead on their own
     shots[1].run(13)
     shots[4].run(40)
@@ -178,15 +179,18 @@ def test_batch_equals_alone(ctx):
             tr, f = outputs(s)
             assert np.array_equal(tr, alone[k][0]), (gs, k)
             assert np.array_equal(f, alone[k][1]), (gs, k)
+        assert (b.graphs()[1] > 0) == (one_step and gs > 0)
         b.close()
 
 
+@pytest.mark.parametrize("one_step", ["none", "all", "every second"])
 @pytest.mark.parametrize("group_kib", [1, 300, 900, 1 << 20])
-def test_grouped_batch_equals_alone(ctx, group_kib):
+def test_grouped_batch_equals_alone(ctx, group_kib, one_step):
     """Shots packed into groups by footprint (budgets below every shot, a
     few shots per group, all shots in one group) and run group after
-    group give the same bits as each shot alone, with and without graph
-    replay, staged and per-lane forms."""
+    group give the same bits as each shot alone: several steps a launch, one
+    step with and without graph replay, staged and per-lane, and groups of
+    either form after groups of the other, whose graphs a new table ends."""
     from seismod_amd.solver import E2dBatch
     rng = np.random.default_rng(31)
     specs = []
@@ -202,7 +206,8 @@ def test_grouped_batch_equals_alone(ctx, group_kib):
         s.run(d["nsteps"])
         alone.append(outputs(s))
         s.close()
-    shots = [make(ctx, d, launch=(2, 0)) for d in dks]
+    shots = [make(ctx, d, launch=(2, 0), one_step=one_step == "all" or (one_step != "none" and k % 2 == 0))
+             for k, d in enumerate(dks)]
     for gs, variant in ((0, "rows"), (8, "staged")):
         for s in shots:
             s.reset()
@@ -210,12 +215,40 @@ def test_grouped_batch_equals_alone(ctx, group_kib):
         b.set_variant(variant)
         b.set_group_bytes(group_kib * 1024)
         b.run(shots, [d["nsteps"] for d in dks])
+        assert (b.graphs()[1] > 0) == (one_step != "none" and gs > 0)
         b.close()
         for k, (s, d) in enumerate(zip(shots, dks)):
             assert s.step == d["nsteps"]
             tr, f = outputs(s)
             assert np.array_equal(tr, alone[k][0]), (gs, k)
             assert np.array_equal(f, alone[k][1]), (gs, k)
+    for s in shots:
+        s.close()
+
+
+def test_graph_cache_is_bounded(ctx):
+    """More stretches of shots than the cache holds graphs for: the least
+    recently used ones go, and a second run gives the same bits."""
+    from seismod_amd.solver import E2dBatch
+    dks = [deck(nx=20 + k, nz=30, npml=4, seed=60 + k, nsteps=16 * (k + 1)) for k in range(20)]
+    shots = [make(ctx, d, one_step=True) for d in dks]
+    want = []
+    for d in dks:
+        s = make(ctx, d)
+        s.run(d["nsteps"])
+        want.append(outputs(s))
+        s.close()
+    b = E2dBatch(ctx, graph_steps=8)
+    for _ in range(2):
+        for s in shots:
+            s.reset()
+        b.run(shots, [d["nsteps"] for d in dks])
+        live, built = b.graphs()
+        assert live == 16 and built >= 20
+        for s, (tr, f) in zip(shots, want):
+            got = outputs(s)
+            assert np.array_equal(got[0], tr) and np.array_equal(got[1], f)
+    b.close()
     for s in shots:
         s.close()
 

@@ -17,8 +17,8 @@ def test_results_alone_equal_results_in_mix(policy):
     assert kinds == {"e2d", "a3d"}
     srv = serve.Server(tick_steps=16, graph_steps=8, policy=policy)
     mix = srv.run(reqs)
-    live, built = srv.batch.graphs()
-    assert live <= min(built, 16)        # the graph cache stays bounded
+    # every 2D shot here takes several steps a launch, which needs no graphs
+    assert srv.batch.graphs() == (0, 0)
     srv.close()
     alone = serve.run_sequential(reqs)
     assert [r.rid for r in mix] == [r.rid for r in alone] == sorted(r.rid for r in reqs)
