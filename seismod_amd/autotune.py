@@ -15,6 +15,10 @@ before the solver's real run.
   2D (Elastic2D):   rows_per_chunk in {1, 2, 3, 4, 6, 8, 12, 16}
   2D batches:       rows_per_chunk and kernel form for the whole batch, then
                     the shot-group budget (tune_e2d_groups)
+
+The 2D rows and forms are those of the one-step launch, which single steps,
+allocation-free batches and solvers without multistep take; runs of two steps
+and more choose their shape by themselves.
 """
 from __future__ import annotations
 
@@ -56,12 +60,15 @@ def _save(path):
     os.replace(tmp, path)
 
 
-def _time(sim, ctx, steps: int) -> float:
+def _time(sim, ctx, steps: int, single: bool = False) -> float:
+    """ms a step over `steps` steps; single: in runs of one step"""
     sim.reset()
-    sim.run(2)
+    for n in (1, 1) if single else (2,):
+        sim.run(n)
     ctx.sync()
     sim.set_timing(True)
-    sim.run(steps)
+    for n in (1,) * steps if single else (steps,):
+        sim.run(n)
     ms, n = sim.timing()
     sim.set_timing(False)
     return ms / max(n, 1)
@@ -111,8 +118,9 @@ def tune_a3d(sim, ctx, steps: int = 8, cache_file=None, candidates=None,
 
 
 def tune_e2d(sim, ctx, steps: int = 20, cache_file=None, candidates=None) -> tuple[int, int]:
-    """Pick rows_per_chunk for an Elastic2D solver (graph steps kept);
-    applies it.  Returns (rows_per_chunk, graph_steps)."""
+    """Pick rows_per_chunk of an Elastic2D solver's one-step launch (graph
+    steps kept), timed in runs of one step; applies it.  Returns
+    (rows_per_chunk, graph_steps)."""
     key = _key_e2d(sim)
     gs = sim.launch()[1]
     with _LOCK:
@@ -126,7 +134,7 @@ def tune_e2d(sim, ctx, steps: int = 20, cache_file=None, candidates=None) -> tup
     best = None
     for c in candidates:
         sim.set_launch(c, 0)
-        t = _time(sim, ctx, steps)
+        t = _time(sim, ctx, steps, single=True)
         if best is None or t < best[0]:
             best = (t, c)
     sim.reset()
@@ -138,14 +146,14 @@ def tune_e2d(sim, ctx, steps: int = 20, cache_file=None, candidates=None) -> tup
 
 
 def tune_e2d_batch(sims, ctx, steps: int = 8, candidates=(1, 2, 3, 4),
-                   variants=("rows", "staged")) -> int:
-    """Pick one rows_per_chunk and kernel form for a batch of Elastic2D
-    solvers advanced together (sm_e2d_batch_run), timing the whole batch;
-    applies the chunk to every solver and resets them.  Many shots in flight favour other chunk lengths
-    than one shot alone: each wave's rows are processed one after another,
-    so the chunk trades waves in flight against the halo rows every chunk
-    recomputes.  Returns (rows_per_chunk, variant); pass the variant to
-    E2dBatch.set_variant."""
+                   variants=("rows", "staged")) -> tuple[int, str]:
+    """Pick one rows_per_chunk and kernel form of the one-step launch for a
+    batch of Elastic2D solvers advanced together, timing the whole batch in
+    runs of one step; applies the chunk to every solver and resets them.  Many
+    shots in flight favour other chunk lengths than one shot alone: each
+    wave's rows are processed one after another, so the chunk trades waves in
+    flight against the halo rows every chunk recomputes.  Returns
+    (rows_per_chunk, variant); pass the variant to E2dBatch.set_variant."""
     from seismod_amd.solver import E2dBatch
     gs = [s.launch()[1] for s in sims]
     best = None
@@ -157,9 +165,12 @@ def tune_e2d_batch(sims, ctx, steps: int = 8, candidates=(1, 2, 3, 4),
                 for s in sims:
                     s.reset()
                     s.set_launch(c, 0)
-                batch.run(sims, [2] * len(sims))
+                one = [1] * len(sims)
+                batch.run(sims, one)
+                batch.run(sims, one)
                 batch.set_timing(True)
-                batch.run(sims, [steps] * len(sims))
+                for _ in range(steps):
+                    batch.run(sims, one)
                 ms, n = batch.timing()
                 batch.set_timing(False)
                 t = ms / max(n, 1)
@@ -173,13 +184,17 @@ def tune_e2d_batch(sims, ctx, steps: int = 8, candidates=(1, 2, 3, 4),
     return best[1], best[2]
 
 
-def tune_e2d_groups(batch, sims, steps: int = 16, candidates_mb=(0, 192, 256, 320, 384)) -> int:
+def tune_e2d_groups(batch, sims, steps=96, candidates_mb=(0, 192, 256, 320, 384)) -> int:
     """Pick the shot-group budget of an E2dBatch (sm_e2d_batch_set_group_bytes):
-    each candidate runs every shot `steps` steps, group after group, timed
-    on the wall clock (groups also save launches, which kernel timing would
-    not show); applies the fastest and resets the solvers.  Returns bytes."""
+    each candidate runs the shots `steps` steps (one number, or one per shot),
+    group after group, timed on the wall clock (groups also save launches,
+    which kernel timing would not show); applies the fastest and resets the
+    solvers.  The steps of a launch are chosen by the steps of a run, so few
+    steps rank the budgets at another kernel shape than a long run's: 16 fit
+    launches of 8, a run of a thousand takes 7.  Returns bytes."""
     import time
     best = None
+    counts = [int(steps)] * len(sims) if not hasattr(steps, "__len__") else list(steps)
     for mb in candidates_mb:
         nbytes = int(mb * 2 ** 20)
         batch.set_group_bytes(nbytes)
@@ -189,7 +204,7 @@ def tune_e2d_groups(batch, sims, steps: int = 16, candidates_mb=(0, 192, 256, 32
         for s in sims:
             s.reset()
         t0 = time.perf_counter()
-        batch.run(sims, [steps] * len(sims))
+        batch.run(sims, counts)
         t = time.perf_counter() - t0
         if best is None or t < best[0]:
             best = (t, nbytes)

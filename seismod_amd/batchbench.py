@@ -6,12 +6,14 @@ plain per-shot launches, on one GPU.
 Workload (seismod_amd.synth.e2d_batch_shots): grids nx ~ U{300..1200} by
 nz ~ U{300..800}, 20-cell PML, 3-6 layers (Vp 2000-5000 m/s, Vs = Vp/1.7-1.9,
 rho 1800-2700), Ricker 10-40 Hz, 1000-3000 steps, dt at half the CFL limit,
-FP32.  Set-up (model upload, autotuning of rows per chunk: per shot for
+FP32.  Set-up (model upload, autotuning of the one-step launch: per shot for
 the plain launches, for the whole batch for the batched run, then of the
 shot-group budget that keeps each group's fields in the last-level cache)
 is outside the timed region; each timed run starts from zero state.  Prints one JSON line:
-aggregate cell-updates per second batched (hipGraph replay) and one shot
-after another with plain launches, and the batch's kernel time per step.
+aggregate cell-updates per second batched and one shot after another, and the
+batch's kernel time per step.  "multistep" says that every shot took several
+steps a launch; rows_per_chunk, kernel_variant and graph_steps shape one-step
+launches only.
 """
 from __future__ import annotations
 
@@ -90,7 +92,8 @@ def main(argv=None) -> None:
            "batched": {"wall_s": round(wall_b, 4), "gcell_updates_per_s": round(work / wall_b / 1e9, 2),
                        "launches": launches, "kernel_ms_per_launch": round(kms / max(launches, 1), 4),
                        "graph_steps": args.graph_steps, "rows_per_chunk": batch_chunk,
-                       "kernel_variant": batch_variant, "group_mb": best_mb,
+                       "kernel_variant": batch_variant,
+                       "multistep": all(s.multistep() for s in sims), "group_mb": best_mb,
                        "by_group_mb": {str(k): round(work / v[0] / 1e9, 2) for k, v in groups.items()}},
            "alg_bytes_per_cell": round(sum(synth.algorithmic_bytes_e2d(sh.nx, sh.nz, sh.npml) * sh.cells * n
                                            for sh, n in zip(shots, steps)) / work, 3)}

@@ -10,8 +10,10 @@ solve with its own model, source, receivers and step count.  The server:
     finishes;
   - advances admitted shots in ticks of `tick_steps` time steps: the 3D
     shots are queued on their own streams first (asynchronous), then the
-    2D shots advance together in one batched launch per time step
-    (sm_e2d_batch_run), so the device works on several shots at once.
+    2D shots advance together in batched launches (sm_e2d_batch_run; of
+    several time steps, or of one, replayed from hipGraphs of graph_steps,
+    while a shot without multistep is among them), so the device works on
+    several shots at once.
     Which shots a tick advances is the policy: "srpt-all" (default) takes
     the admitted shots with the least remaining work (cells x steps left),
     both kinds ranked together, until about one device's worth of cells is
@@ -27,7 +29,7 @@ A shot's result does not depend on what else is running: the kernels give
 the same bits alone, batched, or in any launch shape.
 
 `run_sequential` is the comparison point: one shot at a time in arrival
-order, each with plain per-step launches.
+order, each with plain launches.
 
 CLI:  python -m seismod_amd.serve --rate 20 --count 24 [--seed 5]
           [--policy srpt|srpt-all|share]
@@ -305,7 +307,7 @@ class Server:
 
 
 def run_sequential(requests: list[Request], device: int = 0, keep_traces: bool = True):
-    """One shot at a time in arrival order, plain per-step launches."""
+    """One shot at a time in arrival order, plain launches."""
     ctx = Context(device)
     results = []
     t0 = time.perf_counter()
