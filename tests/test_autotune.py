@@ -98,3 +98,54 @@ def test_e2d_groups_run_the_steps_asked_for():
     assert b.asked == [96, 96, 96]
     autotune.tune_e2d_groups(b, sims, steps=[10, 20, 30], candidates_mb=(0,))
     assert b.asked == [10, 20, 30] and b.group == 0
+
+
+class A3d(Timed):
+    """A flat grid: 15 tiles at 4 rows, 1024 slots, so many chunks are best."""
+
+    class cfg:
+        nx, ny, nz, np, storage = 320, 20, 20, 20, "f32"
+
+    def __init__(self):
+        super().__init__()
+        self.v, self.shape = "cell", (4, 60)
+
+    def variant(self):
+        return self.v
+
+    def set_variant(self, v):
+        if v != self.v:
+            self.v, self.shape = v, (4, 60)
+
+    def launch(self):
+        return self.shape
+
+    def set_launch(self, rows, chunks):
+        length = -(-360 // chunks)
+        if (chunks - 1) * length >= 360:
+            raise ValueError("empty chunk")
+        self.shape = (rows, chunks)
+
+    def run(self, n):
+        rows, chunks = self.shape
+        items = chunks * (60 // rows)
+        self.tick((1.0 if self.v == "tile" else 1.2) * max(1.0, 1024 / items) * (1.1 if rows != 8 else 1.0), n)
+
+
+def test_a3d_tunes_no_worse_than_its_own_launch():
+    s = A3d()
+    for v in ("cell", "tile"):
+        s.set_variant(v)
+        s.reset()
+        s.run(1)
+    own = autotune._time(s, Ctx(), 1)
+    assert autotune.tune_a3d(s, Ctx()) == ("tile",) + s.launch()
+    assert autotune._time(s, Ctx(), 1) <= own
+    # the chunks of 4 rows at 8 rows, as many items: 120 wanted, 60 the most of 6 planes
+    assert s.launch() == (4, 60)
+
+
+def test_a3d_candidates_given_are_the_only_ones():
+    s = A3d()
+    assert autotune.tune_a3d(s, Ctx(), candidates=[(2, 8), (4, 8)], variants=("cell",))[0] == "cell"
+    assert s.launch() in ((2, 8), (4, 8))
