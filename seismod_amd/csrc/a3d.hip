@@ -339,7 +339,6 @@ float half_to_float(uint16_t h)
     return f;
 }
 
-// state values on the host as double, scaled back to physical units
 // rows of n elements, pitch apart, one after the other
 template <typename E>
 __global__ void a3d_pack(const E *src, E *dst, unsigned n, unsigned total, size_t pitch)
@@ -348,11 +347,14 @@ __global__ void a3d_pack(const E *src, E *dst, unsigned n, unsigned total, size_
     if (q < total) dst[q] = src[(size_t)(q / n) * pitch + q % n];
 }
 
-// copies `count` rows of n values, rows `pitch_elems` apart on the device.
+// state values on the host as double, scaled back to physical units: copies
+// `count` rows of n values, rows `pitch_elems` apart on the device.
 // A strided copy to the host goes row by row (400 rows of 340 BF16 cells: 2.8
 // ms, as long as 8 steps), so the fused path packs the rows into the half of
-// its state that the next step overwrites, every cell of it, and copies them
-// in one piece (0.07 ms); the one-half layouts have no such space.
+// its state that the next step overwrites and copies them in one piece (0.07
+// ms); the one-half layouts have no such space.  (The next step writes every
+// cell of the grid; values left in the rows' pad cells, which the cell kernels
+// do not write, are read by no update.)
 int state_to_host(sm_a3d *s, const void *dev, size_t n, size_t count, size_t pitch_elems, float scale, double *out)
 {
     const size_t e = s->elt;

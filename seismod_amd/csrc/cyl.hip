@@ -11,7 +11,7 @@
 // operand order for that region (FP64 storage reproduces it bit for bit;
 // -ffp-contract=off keeps multiply and add separate).  Two launches per
 // step: velocities, then force sources at their cells; stresses, then the
-// Kurkjian source.  Receivers are gathered by a third small kernel.
+// Kurkjian source and the receivers.
 //
 // CPML memory variables exist only where the reference keeps them:
 //   r layers: rows i >= nx-1, (np+1) rows x nz2, index (i-(nx-1))*nz2 + j;
@@ -436,10 +436,10 @@ __device__ __forceinline__ void stress_cell(const CylDev<T> &d, int i, int j)
     }
 }
 
-// receiver values after step it (divergence and curl evaluated at the
-// receiver's cell with propagate.c:4090-4119's expressions; cells outside
-// their ranges read 0 as the reference's zero-initialised arrays do)
-// the recorded value of component comp at padded cell c
+// the recorded value of component comp at padded cell c after step it
+// (divergence and curl evaluated there with propagate.c:4090-4119's
+// expressions; cells outside their ranges read 0 as the reference's
+// zero-initialised arrays do)
 template <typename T>
 __device__ __forceinline__ T recorded(const CylDev<T> &d, int64_t c, int comp)
 {

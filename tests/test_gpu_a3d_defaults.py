@@ -12,9 +12,11 @@ from test_gpu_variants import run
 pytestmark = pytest.mark.gpu
 
 
-# z cells with layers; storage; does a row end at the next cache line
+# z cells with layers; storage; does a row end at a cache line (at most 1/7
+# more cells in 16 bits, 1/16 in FP32) or at a multiple of 8 cells
 PITCH = [(55, "bf16", False), (56, "bf16", True), (57, "f16", True), (58, "bf16", True),
-         (150, "f32", False), (152, "f32", True), (177, "f32", True), (64, "f32", True)]
+         (150, "f32", False), (152, "f32", True), (177, "f32", False), (180, "f32", False), (181, "f32", True),
+         (64, "f32", True)]
 
 
 @pytest.mark.parametrize("nz2,storage,lines", PITCH)
@@ -25,11 +27,16 @@ def test_pitch_equals_forced_lines(ctx, nz2, storage, lines):
     c = d["cfg"]
     need = [A3dConfig(nx=c["nx"], ny=c["ny"], nz=c["nz"], np=np_, dx=c["dx"], dy=c["dy"], dz=c["dz"],
                       dt=c["dt"], f0=c["f0"], storage=storage, sround=s, pad64=p).bytes_needed()
-            for s, p in ((False, False), (False, True), (True, False))]
-    wide = nz2 if nz2 % 64 == 0 else (nz2 // 64 + 1) * 64
-    if wide - nz2 >= 8 and storage != "f32":
-        assert (need[0] == need[1]) == lines
-        assert need[2] < need[1]       # the rounding bits hash the index: their pitch stays
+            for s, p in ((False, False), (False, True), (storage != "f32", False))]
+    # bytes of a cell of pitch: two halves of four fields, three sets of x and y layer arrays, two of material
+    nx2, ny2, e = c["nx"] + 2 * np_, c["ny"] + 2 * np_, 4 if storage == "f32" else 2
+    cell = e * (8 * nx2 * ny2 + 3 * 2 * np_ * (nx2 + ny2)) + 4 * 2 * nx2 * ny2
+    up = lambda q: -(-nz2 // q) * q
+    pitch = [up(64) - (need[1] - n) / cell for n in need]
+    line = 32 if storage == "f32" else 64
+    assert pitch[0] == (up(line) if lines else up(8))
+    # the rounding bits hash the index: with them the limit of 16 bits stays 1/10
+    assert pitch[2] == (pitch[0] if storage == "f32" else up(8) if 10 * (up(64) - nz2) > nz2 else up(64))
     a = run(ctx, d, storage, "tile")
     b = run(ctx, d, storage, "cell", pad64=True)
     assert np.abs(a[0]).max() > 0
