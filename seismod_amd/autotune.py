@@ -201,14 +201,17 @@ def tune_e2d_batch(sims, ctx, steps: int = 8, candidates=(1, 2, 3, 4),
     return best[1], best[2]
 
 
-def tune_e2d_groups(batch, sims, steps=96, candidates_mb=(0, 192, 256, 320, 384)) -> int:
+def tune_e2d_groups(batch, sims, steps=16, candidates_mb=(0, 192, 256, 320, 384)) -> int:
     """Pick the shot-group budget of an E2dBatch (sm_e2d_batch_set_group_bytes):
     each candidate runs the shots `steps` steps (one number, or one per shot),
     group after group, timed on the wall clock (groups also save launches,
     which kernel timing would not show); applies the fastest and resets the
-    solvers.  The steps of a launch are chosen by the steps of a run, so few
-    steps rank the budgets at another kernel shape than a long run's: 16 fit
-    launches of 8, a run of a thousand takes 7.  Returns bytes."""
+    solvers.  The steps of a launch and what a group leaves idle at its end
+    depend on the steps of the run, so the run's own counts rank the budgets
+    as the run does; a few steps are a cheap guess, and many equal ones can
+    mislead (24 shots of 104 to 293 steps, budgets 0 and 384 MiB, ms: own
+    counts 12.5 and 13.0, 16 steps each 1.11 and 1.20, 96 each 6.37 and 6.05).
+    Returns bytes."""
     import time
     best = None
     counts = [int(steps)] * len(sims) if not hasattr(steps, "__len__") else list(steps)

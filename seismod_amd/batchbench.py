@@ -64,7 +64,7 @@ def main(argv=None) -> None:
     batch.set_variant(batch_variant)
     groups = {}
     if args.group_mb == "auto":
-        mbs = [autotune.tune_e2d_groups(batch, sims) / 2 ** 20]
+        mbs = [autotune.tune_e2d_groups(batch, sims, steps) / 2 ** 20]
     else:
         mbs = [float(x) for x in args.group_mb.split(",") if x]
     for mb in mbs:

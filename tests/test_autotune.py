@@ -95,7 +95,7 @@ def test_e2d_groups_run_the_steps_asked_for():
     b = E2dBatch(None)
     b.set_variant("rows")
     autotune.tune_e2d_groups(b, sims, candidates_mb=(0, 256))
-    assert b.asked == [96, 96, 96]
+    assert b.asked == [16, 16, 16]
     autotune.tune_e2d_groups(b, sims, steps=[10, 20, 30], candidates_mb=(0,))
     assert b.asked == [10, 20, 30] and b.group == 0
 
