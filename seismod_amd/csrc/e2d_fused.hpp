@@ -22,9 +22,11 @@
 // on 194 k however little it computes, and a batch streams its whole state per
 // step; now a cell moves once in K steps.  190 x 151 cells,
 // 250 steps: 1.74 -> 0.61 ms; 440^2, 1000 steps: 7.24 -> 2.87 ms; 24 shots of
-// 10 M cells in all: 32.3 -> 14.0 ms.  What bounds it: the layers' arithmetic
-// (320 vector instructions a wave and step, 134 without split fields) and, for
-// batches, the tiles' loads with their halos.
+// 10 M cells in all: 32.3 -> 14.0 ms.  What bounds it: for single shots the
+// chain of steps, two barriers and 320 vector instructions each in the layers
+// (134 without split fields); in a 64-shot batch no unit alone (counters:
+// vector units busy 42%, 2.9 TB/s with the halos, waves waiting 43% of their
+// time).
 #pragma once
 
 #include <hip/hip_runtime.h>

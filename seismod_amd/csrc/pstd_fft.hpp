@@ -17,15 +17,16 @@
 // multiplies and transforms back R contiguous elements in registers: three
 // radices cross LDS four times each way and meet five barriers.
 //
-// What bounds it: vector instructions (about 1500 a transform of 1040 points
-// and wave, two thirds of them butterflies) issued by few waves, and the
-// chain of a workgroup's phases (load, five barriers, store: 10 us).  A
-// launch of 4 derivatives of 1040^2 FP32 takes 19.2 us (1.8 TB/s), of 12
-// derivatives 49 us; the out-of-place Stockham passes before, with runtime
-// loops, root tables in LDS and two buffers, 37.7 and 91.1 us.  Two passes
-// with radices up to 40 measured 29.5 and 54.4 us (195 registers, too few
-// waves), one round per pass instead of a loop over items frees the scalar
-// registers of the roots (54.6 -> 49 us).
+// What bounds it: the chain of a workgroup's phases (load, five barriers,
+// store) in few waves.  Counters, 4 derivatives of 1040^2 FP32: 3 waves a
+// SIMD, all of them resident at once and waiting for 53% of their time; the
+// vector units busy 48% of the launch (1660 instructions a wave), LDS 16%; 12
+// derivatives 46% and 17%, in FP64 20% and 14%.  A launch of 4 derivatives of
+// 1040^2 FP32 takes 19.2 us (1.8 TB/s), of 12 derivatives 49 us; the
+// out-of-place Stockham passes before, with runtime loops, root tables in LDS
+// and two buffers, 37.7 and 91.1 us.  Two passes with radices up to 40 measured
+// 29.5 and 54.4 us (195 registers, too few waves), one round per pass instead
+// of a loop over items frees the scalar registers of the roots (54.6 -> 49 us).
 #pragma once
 
 #include <algorithm>
