@@ -22,9 +22,8 @@
 // launch (pstd_fft.hpp) takes every derivative of a stage along both axes,
 // with one read and one write per value instead of six (forward transform,
 // multiplier pass, inverse transform).  hipFFT remains on request
-// (SM_PSTD_HIPFFT) and for lengths without a plan: factors above 13 and more
-// than 2048 points, or more than 3584 points (FP64 1792) and no radices that
-// 512 threads take in one round.
+// (SM_PSTD_HIPFFT) and for lengths without a plan: above 2048 points those
+// with factors above 13, above 3584 (FP64 1792) some of the others.
 //
 // CPML (pml.c:1959-2106): per stage (fp1, fp23, fp4) and axis the rows b,
 // c at nodes, bh, ch at inner half nodes, bH, cH at outer half nodes; the

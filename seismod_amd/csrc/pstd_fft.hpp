@@ -326,7 +326,10 @@ inline int fft_threads(const FftPlan &p, int P)
 // hand-written transform takes this length.
 //
 // First choice are the cheapest radices with which FFT_THREADS threads take
-// every pass in one round: of 2000 points, none below 4.  A line of at most
+// every pass in one round: of 2000 points, none below 4.  (Lines above
+// FFT_FEWER bytes only if no radices are cheaper: with dearer ones hipFFT's
+// long rows are faster along z, FP64 256 x 2376 322 and 414 us a step, but
+// 256 x 2592 402 and 375, 256 x 3430 497 and 412.)  A line of at most
 // FFT_LOOP bytes that has none takes the cheapest of all and loops (1617 to
 // 3402 points in FP32, 1617 in FP64).  A step of the SH solver, FP32, this
 // loop against hipFFT: 256 x 3000 177 and 301 us, 3000 x 256 183 and 425,
@@ -341,15 +344,17 @@ inline int fft_threads(const FftPlan &p, int P)
 // 77.6 and 36.2 us), a quarter of hipFFT's chirp transforms and their copy
 // passes (469 x 363, FP64, a P-SV stage: 45 against 230 us).  One round of
 // FFT_THREADS threads takes m up to 4096, n up to 2048.
-constexpr size_t FFT_LOOP = 28 * 1024;
+constexpr size_t FFT_LOOP = 28 * 1024, FFT_FEWER = 40 * 1024;
 inline bool fft_plan(int n, size_t elt, FftPlan &p)
 {
     auto one_round = [](int m) { return std::max(2, (m + FFT_THREADS - 1) / FFT_THREADS); };
     p = FftPlan();
     if (n < 2) return false;
     p.m = n;
-    bool ok = fft_radices(n, one_round(n), p);
-    if (!ok && 2 * (size_t)n * elt <= FFT_LOOP) ok = p.loop = fft_radices(n, 2, p);
+    const size_t bytes = 2 * (size_t)n * elt;
+    bool ok = bytes <= FFT_FEWER ? fft_radices(n, one_round(n), p)
+                                 : fft_radices(n, 2, p) && fft_threads(p, 1) <= FFT_THREADS;
+    if (!ok && bytes <= FFT_LOOP) ok = p.loop = fft_radices(n, 2, p);
     if (!ok) {
         double cost = 1e30;
         for (int m = 2 * n - 1; m <= 2 * n + n / 4 + 16; ++m) {

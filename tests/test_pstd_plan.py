@@ -4,7 +4,8 @@ or hipFFT.
 
 A length without a factor above 13 has radices up to 16.  One round of 512
 threads needs every radix to be at least n / 512; a line of at most 28 KiB of
-complex values may also take its passes in several rounds.  A length with
+complex values may also take its passes in several rounds, and one of more
+than 40 KiB has such radices only if they are the cheapest.  A length with
 another factor is padded to at least 2 n - 1 points that one round takes.
 """
 from functools import lru_cache
@@ -34,7 +35,7 @@ def test_path_of_every_length(storage, elt):
     for n in range(2, 5000):
         points, rounds = pstd_plan(n, storage)
         if factors(n, max(2, -(-n // 512))):
-            assert (points, rounds) == (n, 1), n
+            assert (points, rounds) == (n, 1) or (2 * n * elt > 40 * 1024 and points == 0), n
         elif factors(n, 2) and 2 * n * elt <= 28 * 1024:
             assert points == n and rounds > 1, n
         elif n <= 2048:
@@ -50,8 +51,12 @@ def test_ordinary_long_axes():
     for n in (1617, 1944, 2000, 2187, 2662, 3000, 3003, 3159, 3200, 3402):
         assert pstd_plan(n, "f32")[0] == n
     assert pstd_plan(2000, "f32") == (2000, 1) and pstd_plan(3000, "f32") == (3000, 2)
-    for n in (1617, 1694, 1600):
+    for n in (1617, 1694, 1600, 2000, 2376, 2560, 4096):
         assert pstd_plan(n, "f64")[0] == n
+    # long lines whose cheapest radices do not fit one round
+    for n in (2592, 2916, 3430):
+        assert pstd_plan(n, "f64")[0] == 0
+    assert pstd_plan(3430, "f32") == (3430, 1) and pstd_plan(4096, "f32") == (4096, 1)
     for storage, most in (("f32", 3402), ("f64", 1694)):
         for n in range(14, most + 1):
             if smooth(n):
